@@ -548,6 +548,15 @@ int gather_launch(GatherJob& J, void* ws, hipStream_t s) {
   return e == hipSuccess ? MI_OK : hip_fail(e, "qmv launch");
 }
 
+bool aligned(const void* p, size_t n) { return (uintptr_t)p % n == 0; }
+
+// Whether a 32-row launch of the few-row kernel fills the GPU by itself at 8 weight tiles a
+// block (wide shapes, e.g. [14336,4096]).
+bool few_row_fills(int64_t N, int64_t K, int gs, int bits) {
+  mi::QmvmPlan q{};
+  return mi::qmvm_plan(32, (int)N, (int)K, gs, bits, 1, &q) && q.wr >= 8 && q.tiles * q.ks >= 192;
+}
+
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Large-M route of the formats the fused kernels do not decode: dequantize the weight into
@@ -970,6 +979,34 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   static const int dq_min = env_int("MI_QMM_DQGEMM_MIN", 256);
   static const int use_dqgemm = env_int("MI_QMM_DQGEMM", 0);
   static const int prefill_min = env_int("MI_QMM_PREFILL_MIN", 128);
+  // 17..128 rows at gs 64: the mid-row kernel. Up to 32 rows only where a 32-row launch of the
+  // few-row kernel fills the GPU at 8 weight tiles a block and this kernel's blocks are wide
+  // (4-bit [14336,4096] 32 rows 19.3 -> 15.9 us, [4096,14336] 19.0 -> 18.2; elsewhere level or
+  // behind: 8-bit [2048,7168] 10.8 against 11.2, 4-bit [2048,768] 4.7 against 5.3). On those
+  // shapes 33..48 rows run as 32 rows here and the rest on the few-row kernel, so that every
+  // row keeps the bits of the separate calls (30.3 -> 26.9 us at 48 rows; one launch 21.3);
+  // from 49 rows on this kernel alone has them (37.5 -> 21.7 us at 64 rows).
+  static const int use_midm = env_int("MI_QMM_MIDM", 1);
+  mi::MidmPlan mp{};
+  if (use_midm && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 && aligned(x, 16) &&
+      aligned(w, 16) && aligned(scales, 4) && aligned(biases, 4) && aligned(y, 8) &&
+      mi::midm_plan(M, N, K, nb, gs, &mp) && (M > 32 || (mp.wide && few_row_fills(N, K, gs, nb)))) {
+    const int64_t rows = M > 32 && M <= 48 && mp.wide && few_row_fills(N, K, gs, nb) ? 32 : M;
+    mi::MidmParams Q{w, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)x,
+                     (uint16_t*)y, nullptr, (int)rows, (int)N, (int)K, mp.steps, mp.ks};
+    if (mp.part_bytes) {
+      void* data = nullptr;
+      rc = workspace(s, mp.part_bytes, &data);
+      if (rc) return rc;
+      Q.part = (float*)data;
+    }
+    hipError_t e = mi::launch_midm(Q, mp, nb, s);
+    if (e != hipSuccess) return hip_fail(e, "midm launch");
+    if (rows == M) return MI_OK;
+    return mi_quantized_matmul((uint16_t*)y + rows * N, (const uint16_t*)x + rows * K, w, scales,
+                               biases, M - rows, N, K, transpose, group_size, bits, mode, x_dtype,
+                               sb_dtype, stream);
+  }
   if (x_dtype == MI_DTYPE_BFLOAT16 && !use_dqgemm && M >= prefill_min &&
       mi::prefill_supported(M, N, K, nb, gs)) {
     mi::PrefillParams Q{w, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)x,

@@ -109,6 +109,28 @@ hipError_t launch_gmm(const QmvParams& P, int mt, int grid_items, hipStream_t s)
 bool gmm_xs_fits(int64_t K);
 hipError_t launch_gmm_xs(const QmvParams& P, int ns, int grid_items, hipStream_t s);
 
+// Mid-row GEMM (midm*.hip): 17..128 rows of bf16 x, affine 4- and 8-bit weights, gs 64. x and w
+// 16-byte aligned, scales, biases 4-byte, y 8-byte.
+struct MidmParams {
+  const uint32_t* w;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  const uint16_t* x;
+  uint16_t* y;
+  float* part;  // ks > 1: fp32 partials [ks][M][N]
+  int M, N, K;
+  int steps, ks;  // 64-value steps of a wave (even), K ranges over blocks
+};
+struct MidmPlan {
+  bool wide;  // 64-row blocks, else 32-row ones
+  int steps, ks;
+  size_t part_bytes;
+};
+bool midm_plan(int64_t M, int64_t N, int64_t K, int bits, int gs, MidmPlan* out);
+hipError_t launch_midm(const MidmParams& P, const MidmPlan& plan, int bits, hipStream_t s);
+// y = bf16(sum over splits, in split order, of part[split][n]); n a multiple of 4
+hipError_t launch_split_reduce(const float* part, uint16_t* y, int64_t n, int ks, hipStream_t s);
+
 // Decode-width kernel (qmv16.hip): M <= 16 rows per item, 16-row weight tiles.
 int qmv16_mp_for_rows(int rows);
 int qmv16_groups_per_chunk(int bits, int gs);

@@ -439,11 +439,14 @@ hipError_t launch_prefill(const PrefillParams& P, hipStream_t s) {
                  : P.bits == 8 ? launch_bits<8>(P, s)
                                : launch_bits<4>(P, s);
   if (e != hipSuccess || P.ks == 1) return e;
-  const int64_t mn4 = (int64_t)P.M * P.N / 4;
-  int64_t g = (mn4 + 255) / 256;
+  return launch_split_reduce(P.part, P.y, (int64_t)P.M * P.N, P.ks, s);
+}
+
+hipError_t launch_split_reduce(const float* part, uint16_t* y, int64_t n, int ks, hipStream_t s) {
+  const int64_t n4 = n / 4;
+  int64_t g = (n4 + 255) / 256;
   if (g > 8192) g = 8192;
-  hipLaunchKernelGGL(prefill_reduce_kernel, dim3((unsigned)g), dim3(256), 0, s, P.part, P.y, mn4,
-                     P.ks);
+  hipLaunchKernelGGL(prefill_reduce_kernel, dim3((unsigned)g), dim3(256), 0, s, part, y, n4, ks);
   return hipGetLastError();
 }
 

@@ -1,0 +1,75 @@
+"""The mid-row kernel (17..128 rows, affine 4- and 8-bit, groups of 64) against the oracle where
+its tiling can go wrong: row counts around each 32-row tile, output widths that end inside a
+block, K ranges that do not divide into the waves' steps (odd group counts, so a row's scales
+start in the middle of a dword), and splits over blocks."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import BF16_TOL, max_err_ratio, to_dev_bf16, to_dev_u32, to_f64, weights
+import mi_qmm
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 64), (36, 192), (100, 960), (260, 1088), (4096, 128), (128, 7168)]
+
+
+def _run(dev, M, N, K, bits, seed):
+    wq, s, b = weights(1, N, K, bits, 64, seed)
+    x = O.make_x_bf16(M, K, seed + 1)
+    y = mi_qmm.quantized_matmul(to_dev_bf16(x, dev), to_dev_u32(wq[0], dev),
+                                to_dev_bf16(s[0], dev), to_dev_bf16(b[0], dev), True, 64, bits)
+    return x, (wq[0], s[0], b[0]), y
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K", SHAPES)
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
+def test_rows_and_tails(dev, M, N, K, bits):
+    print("CASE", dict(t="midm", M=M, N=N, K=K, bits=bits), flush=True)
+    x, w, y = _run(dev, M, N, K, bits, 100 * M + N)
+    truth = O.qmm_f64(x, *w, 64, bits)
+    err = to_f64(y) - truth
+    assert max_err_ratio(to_f64(y), truth) <= BF16_TOL
+    if M <= 64:
+        # exact codes and fp32 sums: what is left is one bf16 rounding of the result, at most
+        # 2^-9 of a value (2-norm below 2^-9 in all), and fp32 sums 1000 times smaller
+        assert np.linalg.norm(err) <= 2.0 ** -9 * 1.01 * np.linalg.norm(truth)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_rows_are_independent(dev, bits):
+    """Infinite and NaN activations stay in their rows, and scales of the next weight row (read
+    with a row's last group where the K range ends) never reach this one."""
+    M, N, K = 40, 72, 320
+    wq, s, b = weights(1, N, K, bits, 64, 9)
+    x = O.make_x_bf16(M, K, 10)
+    clean = mi_qmm.quantized_matmul(to_dev_bf16(x, dev), to_dev_u32(wq[0], dev), to_dev_bf16(s[0], dev),
+                                    to_dev_bf16(b[0], dev), True, 64, bits)
+    xi = x.copy()
+    xi[3, 5], xi[39, 70] = 0x7F80, 0x7FC0
+    si = s[0].copy()
+    si[41, 0] = 0x7F80
+    y = mi_qmm.quantized_matmul(to_dev_bf16(xi, dev), to_dev_u32(wq[0], dev), to_dev_bf16(si, dev),
+                                to_dev_bf16(b[0], dev), True, 64, bits)
+    rows = [m for m in range(M) if m not in (3, 39)]
+    cols = [n for n in range(N) if n != 41]
+    assert torch.equal(y[rows][:, cols], clean[rows][:, cols])
+    assert not torch.isfinite(y[3].float()).any() and not torch.isfinite(y[39].float()).any()
+
+
+def test_unaligned_pointers_take_another_route(dev):
+    """Views that start off a 16-byte (x, w) or dword (scales) boundary still give the result."""
+    M, N, K = 48, 128, 512
+    x, (wq, s, b), y = _run(dev, M, N, K, 4, 77)
+
+    def off(t, n):
+        buf = torch.empty(t.numel() + n, dtype=t.dtype, device=dev)
+        v = buf[n:].view(t.shape)
+        v.copy_(t)
+        return v
+    X, W, S, B = (to_dev_bf16(x, dev), to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev))
+    truth = O.qmm_f64(x, wq, s, b, 64, 4)
+    for args in ((off(X, 4), W, S, B), (X, off(W, 1), S, B)):
+        assert max_err_ratio(to_f64(mi_qmm.quantized_matmul(*args, True, 64, 4)), truth) <= BF16_TOL
