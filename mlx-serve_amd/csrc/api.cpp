@@ -559,6 +559,26 @@ bool few_row_fills(int64_t N, int64_t K, int gs, int bits) {
 
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
+// The mid-row kernel on its plan (midm_plan), partials in the workspace.
+int run_midm(const void* x, const uint32_t* w, const void* scales, const void* biases, void* y,
+             int64_t M, int64_t N, int64_t K, int fmt, const mi::MidmPlan& pl, hipStream_t s) {
+  mi::MidmParams Q{w, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)x,
+                   (uint16_t*)y, nullptr, (int)M, (int)N, (int)K, pl.steps, pl.ks};
+  if (pl.part_bytes) {
+    void* data = nullptr;
+    const int rc = workspace(s, pl.part_bytes, &data);
+    if (rc) return rc;
+    Q.part = (float*)data;
+  }
+  hipError_t e = mi::launch_midm(Q, pl, fmt, s);
+  return e == hipSuccess ? MI_OK : hip_fail(e, "midm launch");
+}
+
+bool midm_aligned(const void* x, const void* w, const void* scales, const void* biases,
+                  const void* y) {
+  return aligned(x, 16) && aligned(w, 16) && aligned(scales, 4) && aligned(biases, 4) && aligned(y, 8);
+}
+
 // Large-M route of the formats the fused kernels do not decode: dequantize the weight into
 // the workspace as bf16 (`dequant` launches that), then the prefill kernel's bf16-weight
 // instance (prefill.hip, bits = 16). The vendor GEMM (dq_gemm) runs instead only under
@@ -946,6 +966,13 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
       hipError_t e = mi::launch_qmvm(Q, fp, s);
       return e == hipSuccess ? MI_OK : hip_fail(e, "qmvm fp launch");
     }
+    // 33..128 rows: the mid-row kernel, against dequantize + the bf16 GEMM (mxfp4 [14336,4096]
+    // 64 rows 123 -> 17 us, 128 rows 129 -> 26; mxfp8 136 -> 25, 140 -> 33)
+    static const int fp_midm = env_int("MI_QMM_MIDM", 1);
+    mi::MidmPlan mp{};
+    if (fp_midm && M > 32 && M <= 128 && midm_aligned(x, w, scales, nullptr, y) &&
+        mi::midm_plan(M, N, K, 100 + fm, gs, &mp))
+      return run_midm(x, w, scales, nullptr, y, M, N, K, 100 + fm, mp, s);
     static const int fp_any_max = env_int("MI_QMM_ANY_MAX", 8);
     if (M <= fp_any_max) {  // decode rows: straight from the packed codes
       hipError_t e = mi::launch_qmv_any((const uint16_t*)x, w, scales, nullptr, (uint16_t*)y, M,
@@ -988,21 +1015,12 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   // from 49 rows on this kernel alone has them (37.5 -> 21.7 us at 64 rows).
   static const int use_midm = env_int("MI_QMM_MIDM", 1);
   mi::MidmPlan mp{};
-  if (use_midm && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 && aligned(x, 16) &&
-      aligned(w, 16) && aligned(scales, 4) && aligned(biases, 4) && aligned(y, 8) &&
-      mi::midm_plan(M, N, K, nb, gs, &mp) && (M > 32 || (mp.wide && few_row_fills(N, K, gs, nb)))) {
+  if (use_midm && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 && (nb == 4 || nb == 8) &&
+      midm_aligned(x, w, scales, biases, y) && mi::midm_plan(M, N, K, nb, gs, &mp) &&
+      (M > 32 || (mp.wide && few_row_fills(N, K, gs, nb)))) {
     const int64_t rows = M > 32 && M <= 48 && mp.wide && few_row_fills(N, K, gs, nb) ? 32 : M;
-    mi::MidmParams Q{w, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)x,
-                     (uint16_t*)y, nullptr, (int)rows, (int)N, (int)K, mp.steps, mp.ks};
-    if (mp.part_bytes) {
-      void* data = nullptr;
-      rc = workspace(s, mp.part_bytes, &data);
-      if (rc) return rc;
-      Q.part = (float*)data;
-    }
-    hipError_t e = mi::launch_midm(Q, mp, nb, s);
-    if (e != hipSuccess) return hip_fail(e, "midm launch");
-    if (rows == M) return MI_OK;
+    rc = run_midm(x, w, scales, biases, y, rows, N, K, nb, mp, s);
+    if (rc || rows == M) return rc;
     return mi_quantized_matmul((uint16_t*)y + rows * N, (const uint16_t*)x + rows * K, w, scales,
                                biases, M - rows, N, K, transpose, group_size, bits, mode, x_dtype,
                                sb_dtype, stream);
@@ -1083,6 +1101,11 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
     hipError_t e = mi::launch_qmvm(Q, op, s);
     return e == hipSuccess ? MI_OK : hip_fail(e, "qmvm odd-width launch");
   }
+  // 33..128 rows: the mid-row kernel, against dequantize + the bf16 GEMM (6-bit [14336,4096] 64
+  // rows 129 -> 45 us, 128 rows 135 -> 52; 2-bit 110 -> 20, 116 -> 28)
+  if (use_midm && odd_width && M > 32 && M <= 128 && midm_aligned(x, w, scales, biases, y) &&
+      mi::midm_plan(M, N, K, nb, gs, &mp))
+    return run_midm(x, w, scales, biases, y, M, N, K, nb, mp, s);
   static const int any_max = env_int("MI_QMM_ANY_MAX", 8);
   if (odd_width && M <= any_max) {  // decode rows: straight from the packed bitstream
     hipError_t e = mi::launch_qmv_any((const uint16_t*)x, w, scales, (const uint16_t*)biases,

@@ -109,8 +109,9 @@ hipError_t launch_gmm(const QmvParams& P, int mt, int grid_items, hipStream_t s)
 bool gmm_xs_fits(int64_t K);
 hipError_t launch_gmm_xs(const QmvParams& P, int ns, int grid_items, hipStream_t s);
 
-// Mid-row GEMM (midm*.hip): 17..128 rows of bf16 x, affine 4- and 8-bit weights, gs 64. x and w
-// 16-byte aligned, scales, biases 4-byte, y 8-byte.
+// Mid-row GEMM (midm*.hip): up to 128 rows of bf16 x. fmt: affine bits 4 or 8 (gs 64), and from
+// 33 rows 2/3/5/6 (gs 64) and 100 nvfp4, 101 mxfp4, 102 mxfp8 (uint8 scales, no biases). x and
+// w 16-byte aligned, scales and biases 4-byte, y 8-byte.
 struct MidmParams {
   const uint32_t* w;
   const uint16_t* scales;
@@ -126,8 +127,8 @@ struct MidmPlan {
   int steps, ks;
   size_t part_bytes;
 };
-bool midm_plan(int64_t M, int64_t N, int64_t K, int bits, int gs, MidmPlan* out);
-hipError_t launch_midm(const MidmParams& P, const MidmPlan& plan, int bits, hipStream_t s);
+bool midm_plan(int64_t M, int64_t N, int64_t K, int fmt, int gs, MidmPlan* out);
+hipError_t launch_midm(const MidmParams& P, const MidmPlan& plan, int fmt, hipStream_t s);
 // y = bf16(sum over splits, in split order, of part[split][n]); n a multiple of 4
 hipError_t launch_split_reduce(const float* part, uint16_t* y, int64_t n, int ks, hipStream_t s);
 

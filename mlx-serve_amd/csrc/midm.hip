@@ -1,18 +1,27 @@
-// Mid-row quantized GEMM (midm_kernel.h): plan, launch, and the 4-bit instances (the 8-bit
-// ones are in midm_b8.hip).
+// Mid-row quantized GEMM (midm_kernel.h): plan, launch, and the 4-bit instances (the others are in
+// midm_b8.hip, midm_odd.hip and midm_fp.hip).
 #include "midm_kernel.h"
 
 #include <algorithm>
 
 namespace mi {
 namespace midm {
-template hipError_t launch_bits<4>(const MidmParams&, bool, hipStream_t);
-extern template hipError_t launch_bits<8>(const MidmParams&, bool, hipStream_t);
+template hipError_t launch_fmt<4>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<8>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<2>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<3>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<5>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<6>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<100>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<101>(const MidmParams&, bool, hipStream_t);
+extern template hipError_t launch_fmt<102>(const MidmParams&, bool, hipStream_t);
 }  // namespace midm
 
-bool midm_plan(int64_t M, int64_t N, int64_t K, int bits, int gs, MidmPlan* out) {
-  // groups of 64, 4-output stores, 32-bit buffer offsets
-  if ((bits != 4 && bits != 8) || gs != 64 || M < 1 || M > 128 || N < 4 || N % 4 || K % 64 ||
+bool midm_plan(int64_t M, int64_t N, int64_t K, int fmt, int gs, MidmPlan* out) {
+  const int bits = midm::fmt_bits(fmt);
+  const bool ex = fmt == 4 || fmt == 8;
+  // affine groups of 64 (a bias-less mode has its own), 4-output stores, 32-bit offsets
+  if ((fmt < 100 && gs != 64) || M < (ex ? 1 : 33) || M > 128 || N < 4 || N % 4 || K % 64 ||
       M * K * 2 >= ((int64_t)1 << 31) || N * (K * bits / 8) >= ((int64_t)1 << 31) ||
       N >= ((int64_t)1 << 30))
     return false;
@@ -52,9 +61,20 @@ bool midm_plan(int64_t M, int64_t N, int64_t K, int bits, int gs, MidmPlan* out)
   return true;
 }
 
-hipError_t launch_midm(const MidmParams& P, const MidmPlan& pl, int bits, hipStream_t s) {
+hipError_t launch_midm(const MidmParams& P, const MidmPlan& pl, int fmt, hipStream_t s) {
   if (P.ks > 1 && !P.part) return hipErrorInvalidValue;
-  hipError_t e = bits == 8 ? midm::launch_bits<8>(P, pl.wide, s) : midm::launch_bits<4>(P, pl.wide, s);
+  hipError_t e = hipErrorInvalidValue;
+  switch (fmt) {
+    case 2: e = midm::launch_fmt<2>(P, pl.wide, s); break;
+    case 3: e = midm::launch_fmt<3>(P, pl.wide, s); break;
+    case 4: e = midm::launch_fmt<4>(P, pl.wide, s); break;
+    case 5: e = midm::launch_fmt<5>(P, pl.wide, s); break;
+    case 6: e = midm::launch_fmt<6>(P, pl.wide, s); break;
+    case 8: e = midm::launch_fmt<8>(P, pl.wide, s); break;
+    case 100: e = midm::launch_fmt<100>(P, pl.wide, s); break;
+    case 101: e = midm::launch_fmt<101>(P, pl.wide, s); break;
+    case 102: e = midm::launch_fmt<102>(P, pl.wide, s); break;
+  }
   if (e != hipSuccess || P.ks == 1) return e;
   return launch_split_reduce(P.part, P.y, (int64_t)P.M * P.N, P.ks, s);
 }

@@ -3,6 +3,6 @@
 
 namespace mi {
 namespace midm {
-template hipError_t launch_bits<8>(const MidmParams&, bool, hipStream_t);
+template hipError_t launch_fmt<8>(const MidmParams&, bool, hipStream_t);
 }  // namespace midm
 }  // namespace mi

@@ -1,4 +1,5 @@
-// Mid-row quantized GEMM, 17..128 activation rows, affine 4- and 8-bit weights in groups of 64:
+// Mid-row quantized GEMM, 17..128 activation rows, affine weights in groups of 64 (4 and 8 bits;
+// 2, 3, 5 and 6 bits from 33 rows) and nvfp4 / mxfp4 / mxfp8 (from 33 rows):
 //   y[M,N] (bf16) = x[M,K] (bf16) @ dequant(w)[N,K]^T, fp32 accumulation,
 // on v_mfma_f32_32x32x16_bf16 with D[m][n] = x[m][k] W[n][k], so a lane's accumulators all
 // belong to one weight row n = lane % 32 and its scale is one register.
@@ -27,6 +28,10 @@
 // (more rows, where the kernels below already round) operands are bf16(s q + b), as the
 // prefill kernel's: 76 VALU a step and row tile whatever the rows, against 52 + 32 a tile.
 //
+// The bias-less modes use the 4- and 8-bit layouts; code x scale is exact in bf16
+// (code_runs.h), so they need neither epilogue nor rounding. The other widths are one
+// bitstream a row: a lane loads the 4 * bits bytes of its own 32 codes.
+//
 // Steps past a wave's range load through a resource of zero records (zeros, no traffic) and
 // their scales are masked to zero, so any K that is a multiple of 64 runs.
 //
@@ -37,6 +42,7 @@
 #include "mi_common.h"
 #include "qmv_common.h"
 #include "dequant_bf16.h"
+#include "code_runs.h"
 
 namespace mi {
 namespace midm {
@@ -150,13 +156,30 @@ constexpr int midm_younger(int t) {
   return n;
 }
 
-template <int BITS, bool EX, int MT, int WN, int WK, int R, int D>
+// Storage bits of a format: affine bits, or 100 nvfp4, 101 mxfp4, 102 mxfp8.
+constexpr int fmt_bits(int fmt) { return fmt < 100 ? fmt : fmt == 102 ? 8 : 4; }
+
+// 8 codes of OB bits starting `byte` bytes into the lane's dwords -> bf16 pairs of s q + b.
+template <int OB, int byte>
+MI_DEV u32x4_t dequant8_odd(const uint32_t (&d)[OB], float s, float b) {
+  constexpr int i = byte / 4, sh = byte % 4 * 8;
+  const uint64_t v = ((((uint64_t)(i + 1 < OB ? d[i + 1 < OB ? i + 1 : i] : 0u)) << 32) | d[i]) >> sh;
+  auto val = [&](int c) { return fmaf(s, (float)((uint32_t)(v >> (c * OB)) & ((1u << OB) - 1u)), b); };
+  return u32x4_t{pack_bf16x2(val(0), val(1)), pack_bf16x2(val(2), val(3)),
+                 pack_bf16x2(val(4), val(5)), pack_bf16x2(val(6), val(7))};
+}
+
+template <int FMT, bool EX, int MT, int WN, int WK, int R, int D>
 __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
+  constexpr bool FP = FMT >= 100;
+  constexpr int BITS = fmt_bits(FMT);
+  constexpr bool ODD = BITS != 4 && BITS != 8;
+  static_assert(!EX || (!FP && !ODD), "exact codes: affine 4 and 8 bits");
   constexpr int U = 4;  // steps of a unit: the loop body, one load of scales and biases
   constexpr int CS = BITS == 4 ? 2 : 1, DC = D / CS;
   constexpr int XI = 4 * MT / WN;  // x DMA instructions of a wave per step
   static_assert(4 * MT % WN == 0 && U % R == 0 && U % D == 0 && D % CS == 0, "rings");
-  constexpr int WOPS = 2, SOPS = 4;
+  constexpr int WOPS = ODD ? (BITS > 4 ? 2 : 1) : 2, SOPS = !FP ? 4 : FMT == 100 ? 1 : 2;
   constexpr int BN = 32 * WN, BM = 32 * MT;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -183,23 +206,50 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
     const int r = min(n0 + 16 * e + (lane & 15), N - 1);
     wo[e] = (uint32_t)r * rowb + (uint32_t)(s0 * 8 * BITS) + 16 * (h + 2 * ((lane >> 4) & 1));
   }
-  // the row's scales start at any half: dwords from the one that holds the first, shifted
+  // bitstream widths: the lane's own 4 * BITS bytes of row fr
+  const uint32_t wodd =
+      (uint32_t)min(n0 + fr, N - 1) * rowb + (uint32_t)(s0 * 8 * BITS) + (uint32_t)(4 * BITS * h);
+  // A step's scales are one half of the row's run of G halves (one bf16 scale, or two e8m0
+  // bytes; nvfp4: one dword). The run starts at any half: dwords from the one that holds the
+  // first, shifted
   const uint32_t sa = ((uint32_t)min(n0 + fr, N - 1) * (uint32_t)G + (uint32_t)s0) * 2;
-  const uint32_t so = sa & ~3u, ssh = (sa & 2u) * 8u;
+  const uint32_t so = FMT == 100 ? sa * 2 : sa & ~3u, ssh = FMT == 100 ? 0u : (sa & 2u) * 8u;
   const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)P.scales, (short)0, (uint32_t)N * (uint32_t)G * 2, kBufFlags);
+      (void*)P.scales, (short)0, (uint32_t)N * (uint32_t)G * (FMT == 100 ? 4 : 2), kBufFlags);
   const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
       (void*)P.biases, (short)0, (uint32_t)N * (uint32_t)G * 2, kBufFlags);
   unsigned char* ring = smem + kp * (R * MT * 4096);
 
   // t0: first step of a unit (a multiple of U, so ring slots are constants), t: step in it
-  u32x4_t W[DC][2];
+  u32x4_t W[ODD ? 1 : DC][2];
+  uint32_t WO[ODD ? D : 1][ODD ? BITS : 1];
   auto load_w = [&](int t0, int c) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)P.w, (short)0, t0 + CS * c < ns ? wrec : 0u, kBufFlags);
+    if constexpr (ODD) {
+      uint32_t(&d)[BITS] = WO[c % D];
+      const int off = (t0 + c) * 8 * BITS;
+      if constexpr (BITS == 2) {
+        const u32x2_t a = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs, wodd, off, 0));
+        d[0] = a.x, d[1] = a.y;
+      } else if constexpr (BITS == 3) {
+        const auto a = __builtin_amdgcn_raw_buffer_load_b96(rs, wodd, off, 0);
+        d[0] = a[0], d[1] = a[1], d[2] = a[2];
+      } else {
+        const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(rs, wodd, off, 0);
+        d[0] = a.x, d[1] = a.y, d[2] = a.z, d[3] = a.w;
+        if constexpr (BITS == 5) {
+          d[4] = __builtin_amdgcn_raw_buffer_load_b32(rs, wodd + 16, off, 0);
+        } else {
+          const u32x2_t e = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs, wodd + 16, off, 0));
+          d[4] = e.x, d[5] = e.y;
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int e = 0; e < 2; ++e)
-      W[c % DC][e] = __builtin_amdgcn_raw_buffer_load_b128(rs, wo[e], (t0 / CS + c) * 64, 0);
+      W[ODD ? 0 : c % DC][e] = __builtin_amdgcn_raw_buffer_load_b128(rs, wo[e], (t0 / CS + c) * 64, 0);
   };
   auto load_x = [&](int t0, int t) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -208,19 +258,24 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
     for (int j = 0; j < XI; ++j)
       dma16(rs, ring + (t % R) * (MT * 4096) + (wn * XI + j) * 1024, xo[j], (t0 + t) * 128);
   };
-  uint32_t ts[3], tb[3];
+  uint32_t ts[FMT == 100 ? 4 : 3], tb[3];
   auto load_s = [&](int t0) __attribute__((always_inline)) {
-    const uint32_t last = ssh ? so + 8 : kOOB;
-    const u32x2_t a = __builtin_bit_cast(
-        u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(sres, so, t0 * 2, 0));
-    const u32x2_t b = __builtin_bit_cast(
-        u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bres, so, t0 * 2, 0));
-    ts[0] = a.x;
-    ts[1] = a.y;
-    ts[2] = __builtin_amdgcn_raw_buffer_load_b32(sres, last, t0 * 2, 0);
-    tb[0] = b.x;
-    tb[1] = b.y;
-    tb[2] = __builtin_amdgcn_raw_buffer_load_b32(bres, last, t0 * 2, 0);
+    if constexpr (FMT == 100) {
+      const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(sres, so, t0 * 4, 0);
+      ts[0] = a.x, ts[1] = a.y, ts[2] = a.z, ts[3] = a.w;
+    } else {
+      const uint32_t last = ssh ? so + 8 : kOOB;
+      const u32x2_t a = __builtin_bit_cast(
+          u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(sres, so, t0 * 2, 0));
+      ts[0] = a.x, ts[1] = a.y;
+      ts[2] = __builtin_amdgcn_raw_buffer_load_b32(sres, last, t0 * 2, 0);
+      if constexpr (!FP) {
+        const u32x2_t b = __builtin_bit_cast(
+            u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bres, so, t0 * 2, 0));
+        tb[0] = b.x, tb[1] = b.y;
+        tb[2] = __builtin_amdgcn_raw_buffer_load_b32(bres, last, t0 * 2, 0);
+      }
+    }
   };
 
   load_s(0);
@@ -243,19 +298,24 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
   // x fragment of rows 32j.., k-step ks: the 8 values the weight operand of ks covers
   auto xfrag = [&](int t, int j, int ks) -> u32x4_t {
     const int r = 32 * j + fr;
-    const int c = BITS == 4 ? 4 * h + ks : 4 * (ks / 2) + 2 * h + ks % 2;
+    const int c = BITS != 8 ? 4 * h + ks : 4 * (ks / 2) + 2 * h + ks % 2;
     return *reinterpret_cast<const u32x4_t*>(ring + (t % R) * (MT * 4096) + r * 128 +
                                              ((c ^ ((r >> 1) & 7)) << 4));
   };
 #pragma unroll 1
   for (int t0 = 0; t0 < P.steps; t0 += U) {
-    uint32_t sd[2], bd[2];
+    uint32_t sd[FMT == 100 ? 4 : 2], bd[2] = {0u, 0u};
+    if constexpr (FMT == 100) {
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const int g = t0 + 2 * d;  // groups past the range: another row's values, masked out
-      const uint32_t mask = (g < ns ? 0xFFFFu : 0u) | (g + 1 < ns ? 0xFFFF0000u : 0u);
-      sd[d] = __builtin_amdgcn_alignbit(ts[d + 1], ts[d], ssh) & mask;
-      bd[d] = __builtin_amdgcn_alignbit(tb[d + 1], tb[d], ssh) & mask;
+      for (int d = 0; d < 4; ++d) sd[d] = t0 + d < ns ? ts[d] : 0u;
+    } else {
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const int g = t0 + 2 * d;  // steps past the range: another row's values, masked out
+        const uint32_t mask = (g < ns ? 0xFFFFu : 0u) | (g + 1 < ns ? 0xFFFF0000u : 0u);
+        sd[d] = __builtin_amdgcn_alignbit(ts[d + 1], ts[d], ssh) & mask;
+        if constexpr (!FP) bd[d] = __builtin_amdgcn_alignbit(tb[d + 1], tb[d], ssh) & mask;
+      }
     }
     float xs[EX ? MT : 1][U];
     if constexpr (EX) {
@@ -292,21 +352,38 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
           xs[j][t] = a + b;
         }
       }
-      u32x4_t& w0 = W[(t / CS) % DC][0];
-      u32x4_t& w1 = W[(t / CS) % DC][1];
-      if (t % CS == 0) swap16(w0, w1);
-      const float s = t % 2 ? hi_f(sd[t / 2]) : lo_f(sd[t / 2]);
-      const float b = t % 2 ? hi_f(bd[t / 2]) : lo_f(bd[t / 2]);
+      u32x4_t& w0 = W[ODD ? 0 : (t / CS) % DC][0];
+      u32x4_t& w1 = W[ODD ? 0 : (t / CS) % DC][1];
+      if (!ODD && t % CS == 0) swap16(w0, w1);
+      const uint32_t sw = FMT == 100 ? sd[t] : sd[t / 2] >> (16 * (t % 2)) & 0xFFFFu;
+      const float s = FP ? 0.f : __uint_as_float(sw << 16);
+      const float b = FP ? 0.f : t % 2 ? hi_f(bd[t / 2]) : lo_f(bd[t / 2]);
+      // e8m0 byte `i` of the step's two as the exponent field of a float
+      auto e8m0 = [&](int i) { return __uint_as_float((sw >> (8 * i) & 0xFFu) << 23); };
       u32x4_t wq[4];
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        if constexpr (BITS == 4) {
+        if constexpr (ODD) {
+          wq[ks] = ks == 0   ? dequant8_odd<BITS, 0>(WO[t % D], s, b)
+                   : ks == 1 ? dequant8_odd<BITS, BITS>(WO[t % D], s, b)
+                   : ks == 2 ? dequant8_odd<BITS, 2 * BITS>(WO[t % D], s, b)
+                             : dequant8_odd<BITS, 3 * BITS>(WO[t % D], s, b);
+        } else if constexpr (BITS == 4) {
           const uint32_t v = t % 2 ? w1[ks] : w0[ks];
-          wq[ks] = EX ? codes4(v) : dq::dequant8(v, s, b);
+          if constexpr (FMT == 100)  // 16-code groups: bytes 2h and 2h + 1 of the step's four
+            wq[ks] = code_runs::fp4_run_e4m3(
+                v, code_runs::fp_e4m3(sw >> (16 * h + 8 * (ks / 2)) & 0xFFu));
+          else if constexpr (FMT == 101)  // 32-code groups: the lane half's byte
+            wq[ks] = code_runs::fp4_run(v, e8m0(h));
+          else
+            wq[ks] = EX ? codes4(v) : dq::dequant8(v, s, b);
         } else {
           const u32x4_t v = ks / 2 ? w1 : w0;
           const uint32_t d0 = ks % 2 ? v.z : v.x, d1 = ks % 2 ? v.w : v.y;
-          wq[ks] = EX ? codes8(d0, d1) : dequant8_bytes(d0, d1, s, b);
+          if constexpr (FMT == 102)  // 32-code groups: the first two k-steps, the last two
+            wq[ks] = code_runs::fp8_run(d0, d1, e8m0(ks / 2));
+          else
+            wq[ks] = EX ? codes8(d0, d1) : dequant8_bytes(d0, d1, s, b);
         }
         if constexpr (!EX) {
 #pragma unroll
@@ -374,11 +451,12 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
   }
 }
 
-template <int BITS, bool EX, int MT, int WN, int WK, int R>
+template <int FMT, bool EX, int MT, int WN, int WK, int R>
 hipError_t launch_one(const MidmParams& P, hipStream_t s) {
-  constexpr int D = BITS == 4 ? 4 : 2;  // two chunks in flight (8-bit: 20.5 us at 2, 21.6 at 4)
+  // two chunks in flight (8-bit: 20.5 us at 2, 21.6 at 4 steps)
+  constexpr int D = fmt_bits(FMT) == 8 ? 2 : 4;
   constexpr int lds = midm_lds<MT, WN, WK, R>();
-  auto k = midm_kernel<BITS, EX, MT, WN, WK, R, D>;
+  auto k = midm_kernel<FMT, EX, MT, WN, WK, R, D>;
   static bool attr = false;
   if (!attr) {
     hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -390,19 +468,22 @@ hipError_t launch_one(const MidmParams& P, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The instances of one width; block shapes as midm_plan counts them.
-template <int BITS>
-hipError_t launch_bits(const MidmParams& P, bool wide, hipStream_t s) {
+// The instances of one format; block shapes as midm_plan counts them. The other widths and
+// the bias-less modes start at 33 rows (fewer take the few-row kernel).
+template <int FMT>
+hipError_t launch_fmt(const MidmParams& P, bool wide, hipStream_t s) {
+  constexpr bool EX = FMT == 4 || FMT == 8;
   const int mt = (P.M + 31) / 32;
+  if constexpr (EX)
+    if (mt == 1)
+      return wide ? launch_one<FMT, true, 1, 2, 4, 4>(P, s) : launch_one<FMT, true, 1, 1, 8, 4>(P, s);
   if (wide)
-    return mt == 1   ? launch_one<BITS, true, 1, 2, 4, 4>(P, s)
-           : mt == 2 ? launch_one<BITS, true, 2, 2, 4, 4>(P, s)
-           : mt == 3 ? launch_one<BITS, false, 3, 2, 4, 2>(P, s)
-                     : launch_one<BITS, false, 4, 2, 4, 2>(P, s);
-  return mt == 1   ? launch_one<BITS, true, 1, 1, 8, 4>(P, s)
-         : mt == 2 ? launch_one<BITS, true, 2, 1, 4, 4>(P, s)
-         : mt == 3 ? launch_one<BITS, false, 3, 1, 4, 2>(P, s)
-                   : launch_one<BITS, false, 4, 1, 4, 2>(P, s);
+    return mt <= 2   ? launch_one<FMT, EX, 2, 2, 4, 4>(P, s)
+           : mt == 3 ? launch_one<FMT, false, 3, 2, 4, 2>(P, s)
+                     : launch_one<FMT, false, 4, 2, 4, 2>(P, s);
+  return mt <= 2   ? launch_one<FMT, EX, 2, 1, 4, 4>(P, s)
+         : mt == 3 ? launch_one<FMT, false, 3, 1, 4, 2>(P, s)
+                   : launch_one<FMT, false, 4, 1, 4, 2>(P, s);
 }
 
 }  // namespace midm

@@ -73,3 +73,26 @@ def test_unaligned_pointers_take_another_route(dev):
     truth = O.qmm_f64(x, wq, s, b, 64, 4)
     for args in ((off(X, 4), W, S, B), (X, off(W, 1), S, B)):
         assert max_err_ratio(to_f64(mi_qmm.quantized_matmul(*args, True, 64, 4)), truth) <= BF16_TOL
+
+
+@pytest.mark.parametrize("fmt", [2, 3, 5, 6, "nvfp4", "mxfp4", "mxfp8"])
+@pytest.mark.parametrize("N,K", [(36, 192), (260, 1088), (4096, 128), (128, 3584)])
+@pytest.mark.parametrize("M", [33, 64, 65, 128])
+def test_other_formats(dev, fmt, M, N, K):
+    print("CASE", dict(t="midm_fmt", fmt=fmt, M=M, N=N, K=K), flush=True)
+    x = O.make_x_bf16(M, K, M + N)
+    if isinstance(fmt, int):
+        wq, s, b = weights(1, N, K, fmt, 64, 50 + fmt)
+        y = mi_qmm.quantized_matmul(to_dev_bf16(x, dev), to_dev_u32(wq[0], dev), to_dev_bf16(s[0], dev),
+                                    to_dev_bf16(b[0], dev), True, 64, fmt)
+        truth = O.qmm_f64(x, wq[0], s[0], b[0], 64, fmt)
+    else:
+        _, bits, gs = O.FP_MODES[fmt]
+        rng = np.random.default_rng(N + K)
+        wq = O.pack(rng.integers(0, 1 << bits, size=(N, K)).astype(np.uint8), bits)
+        lo, hi = (0x20, 0x48) if fmt == "nvfp4" else (118, 126)
+        sc = rng.integers(lo, hi, size=(N, K // gs)).astype(np.uint8)
+        y = mi_qmm.quantized_matmul(to_dev_bf16(x, dev), to_dev_u32(wq, dev),
+                                    torch.from_numpy(sc).to(dev), None, True, gs, bits, fmt)
+        truth = O.bf16_to_f32(x).astype(np.float64) @ O.dequantize_fp(wq, sc, fmt).astype(np.float64).T
+    assert max_err_ratio(to_f64(y), truth) <= BF16_TOL
