@@ -5,13 +5,20 @@
 // copy in memory before a dense GEMM; here each weight tile is dequantized in registers on
 // its way into the matrix cores and never exists in bf16 outside them.
 //
-// Block: 256 (M) x 256 (N) outputs, 8 waves (two per SIMD), v_mfma_f32_32x32x16_bf16 with
-// D[n][m] = W[n][k] x[m][k]. Per 16-wide k-step a lane supplies 8 consecutive k of one
-// weight row (k in [32h, 32h+32) of the 64-wide step, h = lane/32), dequantized as
-// bf16(s*q + b): q from a scaled fp8 conversion, fma(s, q, b), one rounding to bf16 by
-// v_cvt_pk_bf16_f32, as MLX's GPU qmm rounds the weights it stages. The x fragment of the
-// same k-step is the 16-byte slot 4h+ks of the row. All staging is buffer_load ... lds DMA
+// Block: 256 (M) x 256 (N) outputs, 8 waves (two per SIMD), v_mfma_f32_16x16x32_bf16 with
+// D[n][m] = W[n][k] x[m][k]. In a 64-wide step a lane (row lane % 16, quarter q = lane / 16)
+// holds the 16 values k = 16q .. 16q+15 of its weight rows, dequantized as bf16(s*q + b): q
+// from a scaled fp8 conversion, fma(s, q, b), one rounding to bf16 by v_cvt_pk_bf16_f32, as
+// MLX's GPU qmm rounds the weights it stages; k-step e takes values 8e..8e+7 of each quarter,
+// and the x fragment the 16-byte slot 2q+e of the row. All staging is buffer_load ... lds DMA
 // (no VGPR round trip); the schedule is described at prefill_pp_kernel.
+//
+// What bounds it: the matrix cores at a power-limited clock. On random bf16 operands
+// 16x16x32 sustains 1.96 PF and 32x32x16 1.70 PF (registers only, all CUs; 2.4 and 2.3 PF on
+// zeros), so the smaller shape is taken; with the accumulators in plain VGPRs, since in AGPRs
+// the compiler copied them around these MFMAs (4 moves each). 8192 rows 4-bit, 32x32x16 ->
+// 16x16x32: [14336,4096] 889 -> 805 us, [4096,14336] 822 -> 759 (matrix cores busy 60% / 63% at
+// 1.91 GHz, before 59% / 64% at 1.74).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -24,7 +31,6 @@
 namespace mi {
 namespace {
 
-using qmv_detail::mfma32;
 using qmv_detail::vmcnt_imm;
 using dq::dequant8;
 using dq::pack_bf16x2;
@@ -37,15 +43,15 @@ constexpr int kBufFlags = 0x00020000;   // raw dword access
   __builtin_amdgcn_raw_ptr_buffer_load_lds((rsrc), (__attribute__((address_space(3))) void*)(lds), \
                                            SIZE, (voff), (soff), 0, 0)
 
-// Ping-pong variant: 8 waves, two per SIMD. Wave w owns weight rows [32w, 32w + 32) (one
-// 32-row tile) against all 256 x rows (eight 32-row tiles): 8 accumulators (128
+// Ping-pong variant: 8 waves, two per SIMD. Wave w owns weight rows [32w, 32w + 32) (two
+// 16-row tiles) against all 256 x rows (sixteen tiles): 32 accumulators (128
 // registers), so two waves fit a SIMD, and every weight of the block is dequantized by
 // exactly one wave. (VALU work issued beside another wave's MFMAs delays them, so the
 // dequantize count per MFMA is what this layout minimizes; the price is one 1 KB x
-// fragment read per MFMA, half the LDS read bandwidth of a CU.) Each wave's work on a
+// fragment read per two MFMAs, half the LDS read bandwidth of a CU.) Each wave's work on a
 // 64-wide step is two units: "mem" (its packed weights, scales and biases from LDS,
 // dequantized to the 16 bf16 operand registers of the whole step, and the first x
-// fragments) and "mfma" (the step's 32 MFMAs, the remaining x fragments read as they go).
+// fragments) and "mfma" (the step's 64 MFMAs, the remaining x fragments read as they go).
 // The two groups run the same units half a step apart on staggered barriers: while group
 // 0 issues the matrix ops of step t, group 1 dequantizes step t, then the roles swap, so
 // each SIMD always has one wave feeding the matrix core and one doing the VALU/LDS work.
@@ -96,6 +102,18 @@ MI_DEV u32x4_t dequant8_b8(uint32_t w0, uint32_t w1, float s, float b) {
   return o;
 }
 
+// XOR swizzles of the 16-byte LDS slots by row. A ds_read_b128 pass serves lanes 0-3, 12-15,
+// 20-23 and 24-27 of a half together, so with the MFMA's lane layout (16 rows, quarter
+// q = lane / 16) rows 0-3 and 12-15 of quarter q meet rows 4-11 of quarter q + 1: these keep
+// their slots distinct (x: 8 slots of a 128-byte row, lane slot 2q + e; w: 4 of 64 bytes).
+MI_DEV int xswz(int r) { return (r & 2) | ((r >> 2) & 1) | ((r >> 1) & 4); }
+template <int BITS>
+MI_DEV int wswz(int r) { return BITS == 8 ? 3 * ((r >> 2) & 1) : (r >> 2) & 3; }
+
+MI_DEV f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return mfma16x16x32(as_bf16x8(a), as_bf16x8(b), c);
+}
+
 MI_DEV void wait_vm(int n) {  // s_waitcnt vmcnt(n) for the counts one step can issue
   switch (n) {
     case 0: __builtin_amdgcn_s_waitcnt(vmcnt_imm(0)); break;
@@ -118,7 +136,7 @@ prefill_pp_kernel(PrefillParams P) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2, nq = wave & 3;
-  const int fr = lane & 31, h = lane >> 5;
+  const int fr = lane & 15, q = lane >> 4;
   const int M = P.M, N = P.N, K = P.K, G = K / GS;
   const int mtiles = (M + kBM - 1) / kBM;
   const int mt = blockIdx.x % mtiles, nt = blockIdx.x / mtiles;
@@ -137,22 +155,22 @@ prefill_pp_kernel(PrefillParams P) {
   const __amdgpu_buffer_rsrc_t sbres = __builtin_amdgcn_make_buffer_rsrc(
       (void*)((grp ? P.biases : P.scales) + (size_t)n0 * G), 0, nrows * G * 2, kBufFlags);
   // x: wave w moves tile rows 32w..32w+31 as 4 instructions of 8 rows x 128 B; LDS slot p
-  // of row r holds k-slot p ^ ((r >> 1) & 7).
+  // of row r holds k-slot p ^ xswz(r).
   uint32_t xo[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 32 * wave + 8 * i + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int c = (lane & 7) ^ xswz(r);
     xo[i] = (uint32_t)(min(r, mrows - 1) * K + 8 * c) * 2;
   }
   // packed-weight chunk (2 steps at 4 bits, 1 at 8): wave w moves rows 32w..32w+31 as 2
-  // instructions of 16 rows x 64 B; LDS part p (16 B) of row r holds part p ^ ((r >> 2) & 3)
+  // instructions of 16 rows x 64 B; LDS part p (16 B) of row r holds part p ^ wswz(r)
   // of the row's 64 bytes.
   uint32_t wo[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int r = 32 * wave + 16 * i + (lane >> 2);
-    const int c = (lane & 3) ^ ((r >> 2) & 3);
+    const int c = (lane & 3) ^ wswz<BITS>(r);
     wo[i] = (uint32_t)(min(r, nrows - 1) * rowb + 16 * c);
   }
   // scale (group 0) or bias (group 1) chunk: wave moves rows 64nq..64nq+63 as 4
@@ -163,9 +181,12 @@ prefill_pp_kernel(PrefillParams P) {
     const int r = 64 * nq + 16 * i + (lane >> 2);
     so[i] = (uint32_t)(min(r, nrows - 1) * G * 2 + 4 * (lane & 3));
   }
-  // bf16 weights: lane (fr, h) reads bytes 64h .. 64h+63 of its row's 128 per step
+  // bf16 weights: lane (fr, q) reads bytes 32q .. 32q+31 of its two rows' 128 per step
   u32x4_t wreg[W16 ? 3 : 1][4];
-  const uint32_t w16o = (uint32_t)min(32 * wave + fr, nrows - 1) * (uint32_t)rowb + 64 * h;
+  uint32_t w16o[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+    w16o[a] = (uint32_t)min(32 * wave + 16 * a + fr, nrows - 1) * (uint32_t)rowb + 32 * q;
   // DMA of local step st (x; the weight chunk when st is even; the scale chunk when st
   // starts one; bf16 weights into register slot `slot`). Returns the instructions issued
   // (0 past the last step).
@@ -181,7 +202,7 @@ prefill_pp_kernel(PrefillParams P) {
     if constexpr (W16) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        wreg[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(wres, w16o + 16 * i, k * RB, 0);
+        wreg[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(wres, w16o[i / 2] + 16 * (i % 2), k * RB, 0);
       return n + 4;
     }
     if (BITS == 8 || (st & 1) == 0) {
@@ -202,22 +223,18 @@ prefill_pp_kernel(PrefillParams P) {
     return n;
   };
 
-  f32x16_t acc[8];
+  f32x4_t acc[2][16];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-  // The accumulators go to AGPRs (the clobber makes AGPRs available to the allocator),
-  // so the MFMA C/D traffic stays out of the VGPR file the other wave's VALU work uses.
-  asm volatile("" ::: "a0");
-
-  // x fragment of tile i: row 32 i + fr, k-slot 4h + ks.
-  auto xfrag = [&](int stg, int i, int ks) -> u32x4_t {
-    const int r = 32 * i + fr, c = 4 * h + ks;
+    for (int i = 0; i < 16; ++i) acc[a][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // x fragment of tile i, k-step e: row 16 i + fr, k-slot 2q + e.
+  auto xfrag = [&](int stg, int i, int e) -> u32x4_t {
+    const int r = 16 * i + fr, c = 2 * q + e;
     return *reinterpret_cast<const u32x4_t*>(smem + stg * kPPXStage + r * 128 +
-                                             ((c ^ ((r >> 1) & 7)) << 4));
+                                             ((c ^ xswz(r)) << 4));
   };
-  u32x4_t A[4], X[2][8];
+  u32x4_t A[2][2], X[2][8];  // weight operands [row tile][k-step]; x tiles 8 at a time
   auto mem = [&](int st, auto slot_c) {
     constexpr int slot = decltype(slot_c)::value;
 #pragma unroll
@@ -227,48 +244,54 @@ prefill_pp_kernel(PrefillParams P) {
     const unsigned char* wb =
         smem + kPPWOff + (BITS == 4 ? (st >> 1) & 1 : st % 3) * kPPWChunk;
     const unsigned char* sb = smem + kSOff + ((k / kSP) & 1) * 2 * kPPSChunk;
-    // group of this lane's 32 k within the chunk's 8
-    const int gi = GS == 32 ? 2 * (k % 4) + h : GS == 64 ? k % 8 : (k >> 1) % 8;
-    const int r = 32 * wave + fr;
-    // the lane's 32 codes: 16 B (part 2(st%2) + h) at 4 bits, 32 B (parts 2h, 2h+1) at 8
-    const int part = BITS == 4 ? 2 * (st & 1) + h : 2 * h;
-    const u32x4_t q =
-        *reinterpret_cast<const u32x4_t*>(wb + r * 64 + ((part ^ ((r >> 2) & 3)) << 4));
-    u32x4_t q2 = q;
-    if constexpr (BITS == 8)
-      q2 = *reinterpret_cast<const u32x4_t*>(wb + r * 64 + (((part + 1) ^ ((r >> 2) & 3)) << 4));
-    const uint16_t sv = *reinterpret_cast<const uint16_t*>(sb + r * 16 + 2 * gi);
-    const uint16_t bv = *reinterpret_cast<const uint16_t*>(sb + kPPSChunk + r * 16 + 2 * gi);
-    const float sc = __uint_as_float((uint32_t)sv << 16);
-    const float bp = __uint_as_float((uint32_t)bv << 16);
-    if constexpr (BITS == 4) {
+    // group of this lane's 16 k within the chunk's 8
+    const int gi = GS == 32 ? 2 * (k % 4) + (q >> 1) : GS == 64 ? k % 8 : (k >> 1) % 8;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) A[ks] = dequant8(q[ks], sc, bp);
-    } else {
-      A[0] = dequant8_b8(q.x, q.y, sc, bp);
-      A[1] = dequant8_b8(q.z, q.w, sc, bp);
-      A[2] = dequant8_b8(q2.x, q2.y, sc, bp);
-      A[3] = dequant8_b8(q2.z, q2.w, sc, bp);
+    for (int a = 0; a < 2; ++a) {
+      const int r = 32 * wave + 16 * a + fr;
+      const uint16_t sv = *reinterpret_cast<const uint16_t*>(sb + r * 16 + 2 * gi);
+      const uint16_t bv = *reinterpret_cast<const uint16_t*>(sb + kPPSChunk + r * 16 + 2 * gi);
+      const float sc = __uint_as_float((uint32_t)sv << 16);
+      const float bp = __uint_as_float((uint32_t)bv << 16);
+      if constexpr (BITS == 4) {
+        // the lane's 16 codes: 8 B, half q % 2 of part 2(st%2) + q/2 of the row's 64 bytes
+        const int part = 2 * (st & 1) + (q >> 1);
+        const u32x2_t v = *reinterpret_cast<const u32x2_t*>(
+            wb + r * 64 + ((part ^ wswz<BITS>(r)) << 4) + 8 * (q & 1));
+        A[a][0] = dequant8(v.x, sc, bp);
+        A[a][1] = dequant8(v.y, sc, bp);
+      } else {
+        const u32x4_t v =
+            *reinterpret_cast<const u32x4_t*>(wb + r * 64 + ((q ^ wswz<BITS>(r)) << 4));
+        A[a][0] = dequant8_b8(v.x, v.y, sc, bp);
+        A[a][1] = dequant8_b8(v.z, v.w, sc, bp);
+      }
     }
   };
   auto mfma = [&](int st, auto slot_c) {
     constexpr int slot = decltype(slot_c)::value;
     const int stg = st % kRing;
+    // four parts: k-step u / 2 against x tiles 8(u%2) .. +7
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks < 3) {
+    for (int u = 0; u < 4; ++u) {
+      if (u < 3) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) X[(ks + 1) & 1][i] = xfrag(stg, i, ks + 1);
+        for (int i = 0; i < 8; ++i)
+          X[(u + 1) & 1][i] = xfrag(stg, 8 * ((u + 1) & 1) + i, (u + 1) / 2);
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        acc[i] = mfma32(W16 ? wreg[slot][ks] : A[ks], X[ks & 1][i], acc[i]);
-      // the next k-step's fragment reads go out ahead of this k-step's MFMAs, one read
-      // per MFMA, so their latency hides under the matrix work
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          f32x4_t& c = acc[a][8 * (u & 1) + i];
+          c = mfma16(W16 ? wreg[slot][2 * a + u / 2] : A[a][u / 2], X[u & 1][i], c);
+        }
+      // the next part's fragment reads go out ahead of this part's MFMAs, one read per two
+      // MFMAs, so their latency hides under the matrix work
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
-        if (ks < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (u < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -311,24 +334,21 @@ prefill_pp_kernel(PrefillParams P) {
   if (!grp) __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no DMA may outlive the block
 
-  // epilogue: acc[i] register r is D[n = 32 wave + 8(r/4) + 4h + r%4][m = 32 i + fr]
+  // epilogue: acc[a][i] register r is D[n = 32 wave + 16a + 4q + r][m = 16 i + fr]
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + 32 * i + fr;
+  for (int i = 0; i < 16; ++i) {
+    const int m = m0 + 16 * i + fr;
     if (m >= M) continue;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int n = n0 + 32 * wave + 8 * g + 4 * h;
+    for (int a = 0; a < 2; ++a) {
+      const int n = n0 + 32 * wave + 16 * a + 4 * q;
       if (n >= N) continue;
-      if constexpr (SPLIT) {
-        f32x4_t v = {acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]};
+      const f32x4_t v = acc[a][i];
+      if constexpr (SPLIT)
         *reinterpret_cast<f32x4_t*>(P.part + ((size_t)split * M + m) * N + n) = v;
-      } else {
-        u32x2_t o;
-        o.x = pack_bf16x2(acc[i][4 * g], acc[i][4 * g + 1]);
-        o.y = pack_bf16x2(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-        *reinterpret_cast<u32x2_t*>(P.y + (size_t)m * N + n) = o;
-      }
+      else
+        *reinterpret_cast<u32x2_t*>(P.y + (size_t)m * N + n) =
+            u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }
   }
 }
