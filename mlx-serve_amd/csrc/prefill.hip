@@ -27,6 +27,7 @@
 #include "mi_internal.h"
 #include "qmv_common.h"
 #include "dequant_bf16.h"
+#include "prefill_tiles.h"
 
 namespace mi {
 namespace {
@@ -138,10 +139,8 @@ prefill_pp_kernel(PrefillParams P) {
   const int grp = wave >> 2, nq = wave & 3;
   const int fr = lane & 15, q = lane >> 4;
   const int M = P.M, N = P.N, K = P.K, G = K / GS;
-  const int mtiles = (M + kBM - 1) / kBM;
-  const int mt = blockIdx.x % mtiles, nt = blockIdx.x / mtiles;
-  const int m0 = mt * kBM, n0 = nt * kBN;
-  const int split = blockIdx.y;
+  const TileOf at = tile_of_block((M + kBM - 1) / kBM, (N + kBN - 1) / kBN);
+  const int m0 = at.mt * kBM, n0 = at.nt * kBN, split = at.split;
   const int s0 = split * P.sps;
   const int nsteps = min(P.sps, K / kBK - s0);
   const int mrows = min(kBM, M - m0), nrows = min(kBN, N - n0);
