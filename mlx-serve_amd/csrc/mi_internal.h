@@ -219,10 +219,12 @@ struct PrefillParams {
   float* part;
   int ks, sps;  // K splits and 64-wide steps per split
   int bits;     // 4, 8, or 16 (w holds bf16 [N, K])
+  int bm = 256;  // rows of a tile: 256 (prefill.hip) or 128 (prefill128.hip)
 };
 bool prefill_supported(int64_t M, int64_t N, int64_t K, int bits, int gs);
-size_t prefill_plan(PrefillParams& P);  // fills ks / sps; returns workspace bytes
+size_t prefill_plan(PrefillParams& P);  // fills bm / ks / sps; returns workspace bytes
 hipError_t launch_prefill(const PrefillParams& P, hipStream_t s);
+hipError_t launch_prefill128(const PrefillParams& P, hipStream_t s);  // prefill128.hip
 
 extern std::atomic<int64_t> g_library_gemms;  // dq_gemm calls (blas.cpp)
 

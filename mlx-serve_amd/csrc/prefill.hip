@@ -423,38 +423,47 @@ size_t prefill_plan(PrefillParams& P) {
     return v ? std::atoi(v) : 0;
   }();
   const int steps = P.K / kBK;
-  const int64_t tiles = (int64_t)((P.M + kBM - 1) / kBM) * ((P.N + kBN - 1) / kBN);
-  // K splits: the fewest estimated microseconds over rounds of 256 blocks (one per CU) x
-  // 64-wide steps a split (~2.15 us a step for a 256 x 256 tile), plus each split's fp32
-  // partials written and read back once (~5 TB/s); at least 8 steps a split. Measured at
-  // M=512: gate [14336,4096] 2 splits 27.5% of the bf16 peak (3 splits 20.5%), down
-  // [4096,14336] 8 splits 29.2%.
-  int ks = 1;
-  if (forced_ks > 0) {
-    ks = forced_ks;
-  } else {
-    double best = 1e30;
-    for (int k = 1; k <= std::max(1, steps / 8); ++k) {
-      const int64_t rounds = (tiles * k + 255) / 256;
-      const int sps = (steps + k - 1) / k;
-      const double part_us = k > 1 ? (double)k * P.M * P.N * 8 / 5e6 : 0.0;
-      const double cost = (double)rounds * sps * 2.15 + part_us;
+  // Tile height and K splits: the fewest estimated microseconds, over rounds of 256 blocks
+  // (one per CU) x 64-wide steps a split, plus, for a split, its fp32 partials written and
+  // read back once (~6 TB/s) and the reduce launch. At least 8 steps a split; those of 128-row
+  // tiles are whole 4-step units. Time a step, full grid: 256 x 256 tiles 1.65 us (4 bits and
+  // bf16) and 1.75 (8 bits), 128 x 256 tiles 1.0 (4 bits), 1.15 (8 bits) and 1.3 (bf16). So a
+  // product that fills the chip several times over takes the 256-row tiles, and the 128-row
+  // ones pay where they need fewer splits. Measured, us, 256-row / 128-row tiles, 4 bits:
+  //   [14336,4096]  256 rows 53 / 48   512 81 / 72   700 105 / 116  2003 217 / 245
+  //   [4096,14336]  256 rows 52 / 45   512 72 / 70   700  94 / 110  1024 117 / 123
+  //   [4096,4096]   256 rows 33 / 27   512 40 / 33   1024 52 / 50   2003  80 / 70
+  // 8 bits: [4096,4096] 512 rows 40 / 35, [14336,4096] 700 rows 109 / 139; bf16 weights (with
+  // the dequantize of 6-bit ones): [4096,4096] 256 rows 44 / 37, [14336,4096] 700 143 / 171.
+  double best = 1e30;
+  for (const int bm : {256, 128}) {
+    const int64_t tiles = (int64_t)((P.M + bm - 1) / bm) * ((P.N + kBN - 1) / kBN);
+    const int unit = bm == 128 ? 4 : 1;
+    const double step_us = bm == 128 ? (P.bits == 4 ? 1.0 : P.bits == 8 ? 1.15 : 1.3)
+                                     : (P.bits == 8 ? 1.75 : 1.65);
+    const int k0 = forced_ks > 0 ? std::min(forced_ks, steps) : 1;
+    const int k1 = forced_ks > 0 ? k0 : std::max(1, steps / 8);
+    for (int k = k0; k <= k1; ++k) {
+      const int sps = (steps + k * unit - 1) / (k * unit) * unit;
+      const int ks = (steps + sps - 1) / sps;
+      const double part_us = ks > 1 ? (double)ks * P.M * P.N * 8 / 6e6 + 3.0 : 0.0;
+      const double cost = (double)((tiles * ks + 255) / 256) * sps * step_us + part_us;
       if (cost < best - 1e-9) {
         best = cost;
-        ks = k;
+        P.bm = bm;
+        P.ks = ks;
+        P.sps = sps;
       }
     }
   }
-  ks = std::max(1, std::min(ks, steps));
-  P.sps = (steps + ks - 1) / ks;
-  P.ks = (steps + P.sps - 1) / P.sps;
   return P.ks > 1 ? (size_t)P.ks * P.M * P.N * sizeof(float) : 0;
 }
 
 hipError_t launch_prefill(const PrefillParams& P, hipStream_t s) {
   if (!prefill_supported(P.M, P.N, P.K, P.bits, P.group_size)) return hipErrorNotSupported;
   if (P.ks > 1 && !P.part) return hipErrorInvalidValue;
-  hipError_t e = P.bits == 16 ? launch_bits<16>(P, s)
+  hipError_t e = P.bm == 128    ? launch_prefill128(P, s)
+                 : P.bits == 16 ? launch_bits<16>(P, s)
                  : P.bits == 8 ? launch_bits<8>(P, s)
                                : launch_bits<4>(P, s);
   if (e != hipSuccess || P.ks == 1) return e;
