@@ -530,17 +530,7 @@ int gather_launch(GatherJob& J, void* ws, hipStream_t s) {
       P.item_count = count;
     }
   }
-  // short K with 64-row items: the x-stationary instance, sized for one round of one block a
-  // CU (ns passes of 256 weight rows a block)
-  static const int use_xs = env_int("MI_QMM_GMM_XS", 1);
-  if (J.grouped && use_xs && J.gmm_mt == 2 && !P.dual && !P.swiglu_gate && mi::gmm_xs_fits(P.K)) {
-    const int64_t tiles = (P.N + 255) / 256;
-    const int64_t ns = std::min<int64_t>(
-        tiles, std::max<int64_t>(1, (int64_t)std::ceil(tiles * J.gmm_items / 256.0)));
-    hipError_t e = mi::launch_gmm_xs(P, (int)ns, J.plan.cfg.grid_z, s);
-    return e == hipSuccess ? MI_OK : hip_fail(e, "grouped (x-stationary) launch");
-  }
-  hipError_t e = J.grouped     ? mi::launch_gmm(P, J.gmm_mt, J.plan.cfg.grid_z, s)
+  hipError_t e = J.grouped     ? mi::launch_gmm(P, J.gmm_mt, J.gmm_items, J.plan.cfg.grid_z, s)
                  : J.one_row   ? mi::launch_qmv1(P, J.plan1, J.plan.cfg.grid_z, s)
                  : J.multi_row ? mi::launch_qmvm_gather(P, J.planm, J.plan.cfg.grid_z, s)
                  : J.narrow    ? mi::launch_qmv16(P, J.plan.cfg, s)

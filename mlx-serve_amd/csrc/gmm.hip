@@ -3,34 +3,35 @@
 // segments in src/transformer.zig:14961-15043, gather at :15011), 4-bit affine weights,
 // group size 64, bf16 activations.
 //
-// A work item is a run of sorted pairs with one expert, cut at 32*MT rows (build_items in
-// quant.hip). One block = one item x one 32*WV-row tile of the expert's weight: it streams
-// that weight tile from HBM exactly once and multiplies it by all the item's rows, so an
-// expert with up to 32*MT rows is read once per call whatever its segment length.
+// A work item is a run of sorted pairs with one expert, cut at 32 or 64 rows (build_items in
+// quant.hip). One block = one item x NS tiles of 128 weight rows of its expert (gate + up: 64
+// of either): it streams those weights from HBM exactly once and multiplies them by all the
+// item's rows.
 //
-// Block: WV waves; wave w owns weight rows n0 + 32w .. +31 (one 32-row MFMA tile) against
-// the item's 32*MT rows (MT tiles) of v_mfma_f32_32x32x16_bf16, D[n][m] = W[n][k] x[m][k],
-// with two accumulator sets (even / odd k-steps) so consecutive MFMAs are independent.
-// Per 64-wide step a lane (fr = lane % 32, h = lane / 32) holds 16 packed bytes of its
-// weight row (k in [32h, 32h+32)), dequantized in registers as bf16(s*q + b)
-// (dq::dequant8: no all-ones MFMA and no per-group epilogue); the x fragment of k-step ks
-// is the 16-byte slot 4h+ks of the row.
-// Pipeline, kD steps deep: a step's weight bytes go to a register ring, its gathered x rows
-// to an LDS ring by buffer_load ... lds DMA (rows past the item's end read past the end of
-// x: zeros, no memory traffic), and every 4 steps each lane loads 8 bytes (4 groups) of its
-// row's scales (h = 0) or biases (h = 1), shared across the lane halves by a permlane swap.
-// The loads of step t are issued kD - 1 steps ahead, the x DMA last, so before step t an
-// exact vmcnt (the younger steps' loads only) publishes its x tile; the barrier waits on
-// LDS traffic only. Chunked scale loads matter: one 2-byte load per lane per step made the
-// L2 serve ~7.8 M requests per 113 MB projection and cost 10%.
-// Occupancy: three 4-wave blocks per CU (<= 168 VGPRs, a 4-deep ring of 32 KB) so that a
-// configs[3] T=512 projection's 768 (item, weight tile) blocks run in one round. With two
-// blocks per CU (8-deep ring) the second round ran on half the chip, and every block's first
-// step waited ~5 us behind the whole launch's initial loads (per-block s_memrealtime stamps);
-// a 4-deep ring measured no slower than the 8-deep one. The dequantize of step t + 1 is
-// interleaved with step t's MFMAs (it needs registers only).
+// What bounds it: the weight stream (226 MB a gate + up call of 128 experts, [768,2048]) as far
+// as the arithmetic keeps up: 3.0 TB/s, where a read of the same pieces alone reaches 5.8. When
+// each wave ran barrier, LDS reads, MFMAs and dequantize one after another, the matrix cores
+// were busy 25% and the VALU 46%, at 2.7 TB/s.
+//
+// Block: 4 waves, three blocks a CU; wave w owns 32 weight rows (two 16-row tiles of
+// v_mfma_f32_16x16x32_bf16) against MT 16-row tiles of x. An item that holds at most half of
+// its rows runs as one of half the tiles. Weights, dequantized once as bf16(s*q + b), scales
+// and biases come straight into registers, one 4-step unit ahead: one instruction reads 16
+// rows x 64 contiguous bytes, two steps; one v_permlane32_swap per dword pair gives each lane
+// two dwords of either step, the 8-value runs sb, sb + 1 of the step's eight (sb = 4 (q % 2) +
+// 2 (q / 2) for quarter q = lane / 16). The gathered x rows come by LDS DMA into a ring of
+// four stages (rows past the item's end read past the end of x: zeros, no memory traffic).
+// One barrier a step, before its second k-step, whose MFMAs carry the LDS reads of the next
+// step's first fragments; every MFMA group carries half of the next step's dequantize. Vector
+// memory operations return in order, so "x stage t + 1 has arrived" is an exact vmcnt. A block
+// with several passes (short K) runs them as one stream of steps, so the rings never drain.
+//
+// Measured, us a call, 4 bits, before -> after: gate + up of 128 experts [768,2048], top 8, 64
+// tokens 84.5 -> 74.6, 512 tokens 100 -> 90; 256 experts [2048,7168], 512 tokens 1765 -> 1471;
+// down projections [2048,768] 64 tokens 42.9 -> 37.9, 512 tokens 52.5 -> 54.4 (64 x rows held
+// in LDS then), [2048,1536] (64 experts, top 6) 512 tokens 61 -> 56, [7168,2048] 690 -> 602.
 #include <algorithm>
-#include <type_traits>
+#include <cmath>
 
 #include "dequant_bf16.h"
 #include "mi_common.h"
@@ -45,469 +46,306 @@ using dq::pack_bf16x2;
 using qmv_detail::decode_item;
 using qmv_detail::Item;
 using qmv_detail::item_x_row;
-using qmv_detail::mfma32;
 using qmv_detail::vmcnt_imm;
 
-constexpr int kOOB = 0x7FFFFFF0;  // buffer offset past any x: the load returns 0, no traffic
-constexpr int kD = 4;        // steps in flight: LDS ring of x tiles, register ring of weights
+constexpr uint32_t kOOB = 0x7FFFFFF0u;  // past any x: the load returns 0, no traffic
+constexpr int kRing = 4, kU = 4;         // LDS stages of x; steps of the unrolled unit
+constexpr int kWaves = 4;
 constexpr int kBufFlags = 0x00020000;
 
-MI_DEV u32x4_t ld16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(u32x4_t,
-                            __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
-// 16 bytes per lane from the buffer into LDS at lds + 16 * lane (LDS DMA)
-MI_DEV void dma16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t voff, uint32_t soff) {
+// 64 lanes x 16 bytes into 1 KB of LDS (lane order)
+MI_DEV void dma16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16,
-                                           (int)voff, (int)soff, 0, 0);
+                                           voff, soff, 0, 0);
 }
-MI_DEV u32x2_t ld8(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+MI_DEV f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
+  return mfma16x16x32(as_bf16x8(a), as_bf16x8(b), c);
+}
+// XOR swizzle of the 16-byte slots of a 128-byte x row: the lanes that one pass of a
+// ds_read_b128 serves (rows 0-3 and 12-15 of quarter q, 4-11 of quarter q + 1) fall in
+// distinct banks with the slots of `sb` below.
+MI_DEV int xswz(int r) { return ((r & 2) << 1) | ((r >> 2) & 1) | ((r >> 2) & 2); }
+
+MI_DEV float half_f(uint32_t d, bool up) {
+  return __uint_as_float(up ? d & 0xFFFF0000u : d << 16);
 }
 
-MI_DEV uint32_t xor32_u32(uint32_t v, int lane) {
-  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return (lane & 32) ? r[0] : r[1];
-}
-
-// DUAL (P.dual): the first WV / 2 waves run the gate bank (w, scales, biases) and the others
-// the up bank (w2, scales2, biases2) on the same rows of both and the same x tile; the
+// MODE 0: plain products. 1: y = SwiGLU(P.swiglu_gate, product). 2 (P.dual): the first two waves run the gate bank (w, scales, biases) and the others
+// the up bank (w2, scales2, biases2) on the same rows of both and the same x tiles; the
 // epilogue writes y = SwiGLU(gate, up) through LDS (each product rounded to bf16 first).
-template <int MT, int WV, bool DUAL>
-__global__ void __launch_bounds__(64 * WV, 12 / WV) gmm_kernel(QmvParams P) {
-  constexpr int kWT = DUAL ? WV / 2 : WV;  // waves per weight bank
-  constexpr int R = 32 * MT, kNT = 32 * kWT, kThreads = 64 * WV;
-  // Dynamic LDS: the x ring (kD stages of R rows x 128 B), then the row table. (With a
-  // static array the compiler would drain every load before each LDS read that may alias
-  // an LDS DMA; the waits here are exact and explicit.)
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+// One item of up to 16 * MT rows.
+template <int MT, int MODE>
+MI_DEV void gmm_item(const QmvParams& P, const Item& it, int NS, unsigned char* smem,
+                     const int64_t* rowtab) {
+  constexpr bool DUAL = MODE == 2, staged = MODE != 0;  // staged: results leave through LDS
+  constexpr int kWT = DUAL ? kWaves / 2 : kWaves;  // waves per weight bank
+  constexpr int R = 16 * MT, kNT = 32 * kWT, kThreads = 64 * kWaves;
+  constexpr int XI = MT / 2;  // x DMA instructions of a wave per step
   constexpr int kStage = R * 128;
-  int64_t* rowtab = reinterpret_cast<int64_t*>(smem + kD * kStage);
-  // x DMA instructions per thread per step: R rows x 128 B over kThreads lanes x 16 B
-  constexpr int XU = R * 8 / kThreads;
-  static_assert(XU >= 1 && XU * kThreads == R * 8, "x tile must split evenly over the lanes");
-  constexpr int kN = XU + 1;  // VMEM instructions per step: x DMA and weights (+1 per chunk)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, h = lane >> 5;
+  const int fr = lane & 15, q = lane >> 4;
   const int N = P.N, K = P.K, G = K / 64, nsteps = K / 64;
-  const int n0 = blockIdx.x * kNT;
-  const int n_items = (int)*P.item_count;
-  const int mw = DUAL ? wave % kWT : wave;     // the wave's 32-row tile in its bank
-  const bool up = DUAL && wave >= kWT;          // wave-uniform
-  const uint32_t wrow = (uint32_t)min(n0 + 32 * mw + fr, N - 1);
-  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)P.x, 0, (int)(uint32_t)(P.x_batch * P.M * (int64_t)K * 2), kBufFlags);
+  const int slice0 = blockIdx.x * kNT * NS;
+  const int npass = min(NS, (N - slice0 + kNT - 1) / kNT), total = npass * nsteps;
+  const int mw = DUAL ? wave % kWT : wave;  // the wave's 32 rows in its bank
+  const bool up = DUAL && wave >= kWT;       // wave-uniform
+  const int sb = 4 * (q & 1) + 2 * (q >> 1);
+  const uint32_t rowb = (uint32_t)K / 2;
+  const uint32_t xrec = (uint32_t)(P.x_batch * P.M * (int64_t)K * 2);
 
-  for (int it_i = blockIdx.y; it_i < n_items; it_i += gridDim.y) {
-    const Item it = decode_item(P, it_i);
-    if (it.cnt <= 0) continue;  // block-uniform
-    const uint32_t e = __builtin_amdgcn_readfirstlane(it.expert_ok ? it.expert : 0u);
-    const bool eok = it.expert_ok;
-    if (tid < R) rowtab[tid] = item_x_row(P, it, tid);  // -1 skip, -2 NaN
-    __syncthreads();
-
-    const size_t mat = (size_t)e * (uint32_t)N;
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((up ? P.w2 : P.w) + mat * (uint32_t)(K / 8)), 0, N * (K / 2), kBufFlags);
-    const uint32_t wo = wrow * (uint32_t)(K / 2) + 16 * h;
-    // lane h = 0 loads its row's scales, h = 1 its biases, 4 groups (8 bytes) at a time; a
-    // lane-half swap shares them
-    const uint16_t* sbp = (h ? (up ? P.biases2 : P.biases) : (up ? P.scales2 : P.scales)) +
-                          (mat + wrow) * (uint32_t)G;
-    const int nch = (nsteps + 3) / 4;
-    // x: DMA instruction i of wave w moves rows 8 (XU w + i) .. +7 (8 x 128 B); LDS slot
-    // p of row r holds k-slot p ^ ((r >> 1) & 7). Rows outside the item read past the
-    // end of x (zeros, no memory traffic).
-    uint32_t xo[XU];
+  const uint32_t e = __builtin_amdgcn_readfirstlane(it.expert_ok ? it.expert : 0u);
+  const bool eok = it.expert_ok;
+  // acc[a][i] register r is D[n = 32 mw + 16 a + 4 q + r][m = 16 i + fr]
+  f32x4_t acc[2][MT];
+  auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < XU; ++i) {
-      const int r = 8 * (XU * wave + i) + (lane >> 3);
-      const int c = (lane & 7) ^ ((r >> 1) & 7);
-      const int64_t ro = rowtab[r];
-      xo[i] = ro >= 0 ? (uint32_t)ro * 2u + 16u * c : (uint32_t)kOOB;
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[a][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  auto store = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = 16 * i + fr;
+      const int64_t ro = rowtab[m];
+      if (ro == -1) continue;
+      const int64_t pos = it.pos0 + m;
+      const bool nan = ro == -2 || !eok;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int n = slice0 + p * kNT + 32 * mw + 16 * a + 4 * q;
+        if (n >= N) continue;
+        u32x2_t o = {pack_bf16x2(acc[a][i][0], acc[a][i][1]),
+                     pack_bf16x2(acc[a][i][2], acc[a][i][3])};
+        if (nan) o = u32x2_t{0x7FC07FC0u, 0x7FC07FC0u};
+        *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = o;
+      }
     }
-
-    u32x4_t wq[kD];
-    u32x2_t sbc[4];  // scale/bias chunks: chunk c (steps 4c..4c+3) in slot c % 4
-    // Step t's loads: its scale chunk when t starts one, its weights, then (last, so the
-    // wait before a step counts only younger loads) its x DMA.
-    auto issue = [&](int t, int slot, int cslot) __attribute__((always_inline)) {
-      const uint32_t tt = (uint32_t)min(t, nsteps - 1);
-      if ((t & 3) == 0)
-        sbc[cslot] = *reinterpret_cast<const u32x2_t*>(sbp + 4 * min(t >> 2, nch - 1));
-      wq[slot] = ld16(wres, wo, tt * 32u);
-      __builtin_amdgcn_sched_barrier(0);
+  };
+  if (!eok) {
+    if (!staged)
+      for (int p = 0; p < npass; ++p) store(p);
+  } else {
+    const size_t mat = (size_t)e * (uint32_t)N;
+    const unsigned char* wb = (const unsigned char*)(up ? P.w2 : P.w) + mat * rowb;
+    const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((up ? P.scales2 : P.scales) + mat * (uint32_t)G), (short)0, N * G * 2, kBufFlags);
+    const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((up ? P.biases2 : P.biases) + mat * (uint32_t)G), (short)0, N * G * 2, kBufFlags);
+    // x: instruction j of wave w moves rows 8 (XI w + j) .. +7. Rows outside the item read
+    // past the end of x (zeros, no memory traffic).
+    uint32_t xo[XI];
 #pragma unroll
-      for (int i = 0; i < XU; ++i)
-        dma16(xres, smem + slot * kStage + (XU * wave + i) * 1024, xo[i], tt * 128u);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int j = 0; j < XI; ++j) {
+      const int r = 8 * (XI * wave + j) + (lane >> 3), c = (lane & 7) ^ xswz(r);
+      const int64_t ro = rowtab[r];
+      xo[j] = ro >= 0 ? (uint32_t)ro * 2u + 16u * c : kOOB;
+    }
+    // flat steps 0 .. total - 1, pass p = step / nsteps (a unit lies in one pass)
+    auto load_w = [&](int p, int t, bool in, int a, u32x4_t& d) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)wb, (short)0, in ? N * rowb : 0u, kBufFlags);
+      const uint32_t r = (uint32_t)min(slice0 + p * kNT + 32 * mw + 16 * a + fr, N - 1);
+      d = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, r * rowb + 16 * q, t * 32, 0));
     };
+    auto load_x = [&](int t, bool in, int slot, int j) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)P.x, (short)0, in ? xrec : 0u, kBufFlags);
+      dma16(rs, smem + slot * kStage + (wave * XI + j) * 1024, xo[j], t * 128);
+    };
+    u32x2_t ts[2], tb[2], sd[2], bd[2];
+    auto load_s = [&](int p, int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const uint32_t r = (uint32_t)min(slice0 + p * kNT + 32 * mw + 16 * a + fr, N - 1);
+        ts[a] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(sres, r * G * 2, t * 2, 0));
+        tb[a] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(bres, r * G * 2, t * 2, 0));
+      }
+    };
+    u32x4_t W[2][2];  // chunk of two steps, row tile
+    // a chunk's dwords to step order: {even step: 2, odd step: 2}
+    auto prep_w = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        u32x4_t& v = W[c][a];
+        const auto x = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+        v = u32x4_t{x[0], y[0], x[1], y[1]};
+      }
+    };
+    auto dq_w = [&](int t, int a, int k) __attribute__((always_inline)) {
+      return dequant8(W[(t / 2) % 2][a][2 * (t % 2) + k], half_f(sd[a][t / 2], t % 2),
+                      half_f(bd[a][t / 2], t % 2));
+    };
+    auto xfrag = [&](int t, int i, int k) -> u32x4_t {
+      return *reinterpret_cast<const u32x4_t*>(smem + (t % kRing) * kStage + (16 * i + fr) * 128 +
+                                               (((sb + k) ^ xswz(fr)) << 4));
+    };
+    // Prologue in the order that the loop's wait counts: the second chunk comes after the
+    // first half of stage 1, as in the loop's step -1.
+    load_s(0, 0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) load_w(0, 0, true, a, W[0][a]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < XI; ++j) load_x(t, true, t, j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) load_w(0, 2, true, a, W[1][a]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_x(2, true, 2, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(XI + 2 + 1));  // stage 0 has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4_t X[2][MT], A[2][2][2];  // fragments of a k-step; operands of this step and the next
+#pragma unroll
+    for (int i = 0; i < MT; ++i) X[0][i] = xfrag(0, i, 0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) sd[a] = ts[a], bd[a] = tb[a];
+    prep_w(0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) A[0][a][k] = dq_w(0, a, k);
+    int pass = 0, tc = 0;  // of the unit
+#pragma unroll 1
+    for (int t0 = 0; t0 < total; t0 += kU) {
+      const bool wrap = tc + kU == nsteps, in = t0 + kU < total;
+      const int pn = in && wrap ? pass + 1 : pass, tn0 = wrap ? 0 : tc + kU;  // next unit
+#pragma unroll
+      for (int t = 0; t < kU; ++t) {
+        const int tn = t + 1;
+        if (tn == kU) {
+#pragma unroll
+          for (int a = 0; a < 2; ++a) sd[a] = ts[a], bd[a] = tb[a];
+        }
+        if (tn % 2 == 0) prep_w((tn / 2) % 2);
+        auto stage = [&](int st, int j) __attribute__((always_inline)) {
+          if (st < kU)
+            load_x(tc + st, true, st % kRing, j);
+          else
+            load_x(tn0 + st - kU, in, st % kRing, j);
+        };
+        // two groups, one k-step each
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          if (u == 1) {
+            // this wave's part of x stage t + 1 is in: younger are the x DMA since (XI),
+            // two weight loads every second step and four scale loads every fourth
+            if (t < 2)
+              __builtin_amdgcn_s_waitcnt(vmcnt_imm(XI + 6));
+            else
+              __builtin_amdgcn_s_waitcnt(vmcnt_imm(XI + 2));
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            stage(t + 3, 0);  // slot of stage t - 1: every wave is past its last read
+          } else {
+            if constexpr (XI > 1) stage(t + 2, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t == 0) load_s(pn, tn0);
+            if (t % 2 == 1) {
+#pragma unroll
+              for (int a = 0; a < 2; ++a) load_w(pn, tn0 + t - 1, in, a, W[t / 2][a]);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < MT; ++i) X[(u + 1) & 1][i] = xfrag(u ? tn : t, i, (u + 1) & 1);
+#pragma unroll
+          for (int a = 0; a < 2; ++a) A[tn & 1][a][u] = dq_w(tn % kU, a, u);
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) acc[a][i] = mfma16(A[t & 1][a][u], X[u][i], acc[a][i]);
+#pragma unroll
+          for (int m = 0; m < 2 * MT; ++m) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (m % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 48 / (2 * MT), 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if (wrap && !staged) {
+        store(pass);
+        clear();
+      }
+      pass = pn;
+      tc = tn0;
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no DMA may outlive its stage
+  }
+  const int n0 = slice0;
 
-    f32x16_t acc[MT];
+  // results through LDS (the x ring's memory), then every thread takes 4 adjacent outputs of
+  // a row: coalesced gate reads and output writes
+  if constexpr (staged) {
+    // DUAL: gate products in columns [0, kNT), up products in [kNT, 2 kNT); row stride
+    // padded by 4 halves
+    constexpr int kTS = (DUAL ? 2 : 1) * kNT + 4;
+    uint16_t* tile = reinterpret_cast<uint16_t*>(smem);
+    __syncthreads();  // every wave is done reading the x ring
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-
-    if (eok) {
-      // step t: wait for its DMA (issued kD - 1 steps earlier) and for step t + 1's weights,
-      // barrier, then the MFMAs of step t with step t + 1's dequantize interleaved (it needs
-      // registers only: the weight ring and the scale chunk), then issue step t + kD - 1
-      // into the stage step t - 1 freed. Unrolled by 16 (four scale chunks) so every
-      // register slot is static.
-#pragma unroll
-      for (int j = 0; j < kD - 1; ++j) issue(j, j, (j >> 2) & 3);
-      // step j's scale and bias (group j % 4 of chunk slot (j / 4) % 4)
-      auto scale_bias = [&](int j, float& sc, float& bp) __attribute__((always_inline)) {
-        const u32x2_t mine = sbc[(j >> 2) & 3];
-        const uint32_t mw = (j & 2) ? mine.y : mine.x;
-        const uint32_t ow = xor32_u32(mw, lane);
-        const uint32_t sw = h ? ow : mw, bw = h ? mw : ow;
-        sc = __uint_as_float((j & 1) ? (sw & 0xFFFF0000u) : (sw << 16));
-        bp = __uint_as_float((j & 1) ? (bw & 0xFFFF0000u) : (bw << 16));
-      };
-      u32x4_t A[4];
-      {
-        // step 0's weights and scale chunk: everything after them may stay in flight
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(XU + (kD - 2) * kN + (kD - 2) / 4));
-        float sc, bp;
-        scale_bias(0, sc, bp);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) A[ks] = dequant8(wq[0][ks], sc, bp);
-      }
-      for (int t0 = 0; t0 < nsteps; t0 += 16) {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int t = t0 + j, js = j % kD;
-          // Done: every load of step t and step t + 1's scale chunk and weights. In flight:
-          // step t + 1's x DMA and steps t + 2 .. t + kD - 2 (kN each plus one per scale
-          // chunk they start). The barrier waits on LDS traffic only.
-          constexpr int kAfter0 = XU + (kD - 3) * kN;
-          const int starts = ((j + kD - 2) >> 2) - ((j + 1) >> 2);  // multiples of 4 in j+2..j+kD-2
-          switch (starts) {
-            case 0: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kAfter0)); break;
-            case 1: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kAfter0 + 1)); break;
-            default: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kAfter0 + 2)); break;
-          }
-          qmv_detail::lds_barrier();
-          if (t < nsteps) {
-            u32x4_t X[4][MT], An[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-              for (int i = 0; i < MT; ++i) {
-                const int r = 32 * i + fr, c = 4 * h + ks;
-                X[ks][i] = *reinterpret_cast<const u32x4_t*>(
-                    smem + js * kStage + r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
-              }
-            float sc, bp;
-            scale_bias(j + 1, sc, bp);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) An[ks] = dequant8(wq[(j + 1) % kD][ks], sc, bp);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-              for (int i = 0; i < MT; ++i)
-                acc[i] = mfma32(A[ks], X[ks][i], acc[i]);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) A[ks] = An[ks];
-            // fragment reads first, then each MFMA with a slice of the next dequantize
-            __builtin_amdgcn_sched_group_barrier(0x100, 4 * MT, 0);
-#pragma unroll
-            for (int m = 0; m < 4 * MT; ++m) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-              __builtin_amdgcn_sched_group_barrier(0x002, 84 / (4 * MT), 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          issue(t + kD - 1, (j + kD - 1) % kD, ((j + kD - 1) >> 2) & 3);
-        }
-      }
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no DMA may outlive its stage
-    }
-
-    // epilogue: acc[i] register r is D[n = 32 mw + 8(r/4) + 4h + r%4][m = 32 i + fr]
-    if constexpr (DUAL) {
-      // gate products in columns [0, kNT) of an LDS tile, up products in [kNT, 2 kNT) (row
-      // stride padded by 4 halves), then every thread takes 4 adjacent outputs of a row
-      constexpr int kTS = 2 * kNT + 4;
-      uint16_t* tile = reinterpret_cast<uint16_t*>(smem);
-      __syncthreads();  // every wave is done reading the x ring
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          u32x2_t o;
-          o.x = pack_bf16x2(acc[i][4 * g], acc[i][4 * g + 1]);
-          o.y = pack_bf16x2(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-          *reinterpret_cast<u32x2_t*>(tile + (32 * i + fr) * kTS + (up ? kNT : 0) + 32 * mw +
-                                      8 * g + 4 * h) = o;
-        }
-      __syncthreads();
-      constexpr int kPerRow = kNT / 4, kRowsPerPass = kThreads / kPerRow;
-      const int c4 = tid % kPerRow;
-      const int n = n0 + 4 * c4;
+      for (int a = 0; a < 2; ++a)
+        *reinterpret_cast<u32x2_t*>(tile + (16 * i + fr) * kTS + (up ? kNT : 0) + 32 * mw + 16 * a +
+                                    4 * q) =
+            u32x2_t{pack_bf16x2(acc[a][i][0], acc[a][i][1]), pack_bf16x2(acc[a][i][2], acc[a][i][3])};
+    __syncthreads();
+    constexpr int kPerRow = kNT / 4, kRowsPerPass = kThreads / kPerRow;
+    const int c4 = tid % kPerRow;
+    const int n = n0 + 4 * c4;
 #pragma unroll 1
-      for (int m = tid / kPerRow; m < R; m += kRowsPerPass) {
-        const int64_t ro = rowtab[m];
-        if (ro == -1 || n >= N) continue;
-        const int64_t pos = it.pos0 + m;
-        u32x2_t gv = *reinterpret_cast<const u32x2_t*>(tile + m * kTS + 4 * c4);
-        u32x2_t uv = *reinterpret_cast<const u32x2_t*>(tile + m * kTS + kNT + 4 * c4);
-        if (ro == -2 || !eok) gv.x = gv.y = uv.x = uv.y = 0x7FC07FC0u;  // NaN rows
-        const uint32_t gw[2] = {gv.x, gv.y}, uw[2] = {uv.x, uv.y};
-        uint32_t o[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const uint32_t lo = swiglu_bf16((uint16_t)(gw[q] & 0xFFFFu), (uint16_t)(uw[q] & 0xFFFFu));
-          const uint32_t hi = swiglu_bf16((uint16_t)(gw[q] >> 16), (uint16_t)(uw[q] >> 16));
-          o[q] = lo | (hi << 16);
-        }
-        u32x2_t ov;
-        ov.x = o[0];
-        ov.y = o[1];
-        *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = ov;
+    for (int m = tid / kPerRow; m < R; m += kRowsPerPass) {
+      const int64_t ro = rowtab[m];
+      if (ro == -1 || n >= N) continue;
+      const int64_t pos = it.pos0 + m;
+      u32x2_t pv = *reinterpret_cast<const u32x2_t*>(tile + m * kTS + 4 * c4), gv = pv;
+      if constexpr (DUAL)
+        pv = *reinterpret_cast<const u32x2_t*>(tile + m * kTS + kNT + 4 * c4);
+      else
+        gv = *reinterpret_cast<const u32x2_t*>(P.swiglu_gate + pos * N + n);
+      if (ro == -2 || !eok) {  // NaN rows
+        pv.x = pv.y = 0x7FC07FC0u;
+        if constexpr (DUAL) gv = pv;
       }
-    } else if (P.swiglu_gate) {
-      // SwiGLU epilogue through LDS: the bf16 products go to a [R][kNT] tile in the x ring
-      // (row stride kNT + 4 halves, so the 32 rows one store instruction covers fall in
-      // distinct banks), the accumulators die, and every thread then takes 4 adjacent
-      // outputs of a row: coalesced gate reads and output writes, and the SwiGLU math
-      // runs with the loop's registers free.
-      constexpr int kTS = kNT + 4;
-      uint16_t* tile = reinterpret_cast<uint16_t*>(smem);
-      __syncthreads();  // every wave is done reading the x ring
+      uint32_t o[2];
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          u32x2_t o;
-          o.x = pack_bf16x2(acc[i][4 * g], acc[i][4 * g + 1]);
-          o.y = pack_bf16x2(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-          *reinterpret_cast<u32x2_t*>(tile + (32 * i + fr) * kTS + 32 * mw + 8 * g + 4 * h) = o;
-        }
-      __syncthreads();
-      constexpr int kPerRow = kNT / 4, kRowsPerPass = kThreads / kPerRow;
-      const int c4 = tid % kPerRow;
-      const int n = n0 + 4 * c4;
-#pragma unroll 1
-      for (int m = tid / kPerRow; m < R; m += kRowsPerPass) {
-        const int64_t ro = rowtab[m];
-        if (ro == -1 || n >= N) continue;
-        const int64_t pos = it.pos0 + m;
-        const u32x2_t gt = *reinterpret_cast<const u32x2_t*>(P.swiglu_gate + pos * N + n);
-        u32x2_t pv = *reinterpret_cast<const u32x2_t*>(tile + m * kTS + 4 * c4);
-        if (ro == -2 || !eok) pv.x = pv.y = 0x7FC07FC0u;  // NaN rows, as the plain path
-        const uint32_t gw[2] = {gt.x, gt.y}, pw[2] = {pv.x, pv.y};
-        uint32_t o[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const uint32_t lo = swiglu_bf16((uint16_t)(gw[q] & 0xFFFFu), (uint16_t)(pw[q] & 0xFFFFu));
-          const uint32_t hi = swiglu_bf16((uint16_t)(gw[q] >> 16), (uint16_t)(pw[q] >> 16));
-          o[q] = lo | (hi << 16);
-        }
-        u32x2_t ov;
-        ov.x = o[0];
-        ov.y = o[1];
-        *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = ov;
+      for (int d = 0; d < 2; ++d) {
+        const uint32_t lo = swiglu_bf16((uint16_t)(gv[d] & 0xFFFFu), (uint16_t)(pv[d] & 0xFFFFu));
+        const uint32_t hi = swiglu_bf16((uint16_t)(gv[d] >> 16), (uint16_t)(pv[d] >> 16));
+        o[d] = lo | (hi << 16);
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = 32 * i + fr;
-        const int64_t ro = rowtab[m];
-        if (ro == -1) continue;
-        const int64_t pos = it.pos0 + m;
-        const bool nan = ro == -2 || !eok;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = n0 + 32 * mw + 8 * g + 4 * h;
-          if (n >= N) continue;
-          float v[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = nan ? __builtin_nanf("") : acc[i][4 * g + q];
-          u32x2_t o;
-          o.x = pack_bf16x2(v[0], v[1]);
-          o.y = pack_bf16x2(v[2], v[3]);
-          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = o;
-        }
-      }
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = u32x2_t{o[0], o[1]};
     }
-    __syncthreads();  // the row table and the x ring are reused by the next item
   }
+  __syncthreads();  // the row table and the x ring are reused by the next item
 }
 
-// x-stationary variant for short K: the item's 64 x rows, all of K, fit in LDS, so the block
-// moves them once by LDS DMA and then streams NS passes of 32 WV weight rows each (the
-// wave's 32 rows of every pass, one after another through one register ring) with no
-// barrier and no DMA inside the loop. Row r of x sits at r * S (S = 2K bytes rounded up to
-// 1 KB, one DMA instruction's span, plus 128 B so that consecutive rows start half the banks
-// apart), k-step t at + 128 t, and slot p of a step holds k-slot p ^ ((r >> 1) & 7), as in
-// the ring layout of gmm_kernel.
-__host__ __device__ constexpr int xs_row_stride(int K) { return (K * 2 + 1023) / 1024 * 1024 + 128; }
-#ifndef MI_GMM_XS_DEPTH
-#define MI_GMM_XS_DEPTH 8
-#endif
-constexpr int kXsD = MI_GMM_XS_DEPTH;  // weight ring depth of the x-stationary kernel
-static_assert(kXsD == 4 || kXsD == 8 || kXsD == 16, "the step loop unrolls by 16");
-
-template <int WV>
-__global__ void __launch_bounds__(64 * WV, 1) gmm_xs_kernel(QmvParams P, int NS) {
-  constexpr int MT = 2, R = 64, kNT = 32 * WV;
+// Items of 16 * MT rows; one that holds at most half of them runs as such.
+template <int MT, int MODE>
+__global__ void __launch_bounds__(64 * kWaves, 3) gmm_kernel(QmvParams P, int NS) {
+  // Dynamic LDS: the x ring, then the row table. (With a static array the compiler would
+  // drain every load before each LDS read that may alias an LDS DMA; the waits here are
+  // exact and explicit.)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int N = P.N, K = P.K, G = K / 64, nsteps = K / 64;
-  const int S = xs_row_stride(K);
-  int64_t* rowtab = reinterpret_cast<int64_t*>(smem + R * S);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, h = lane >> 5;
+  int64_t* rowtab = reinterpret_cast<int64_t*>(smem + kRing * 16 * MT * 128);
   const int n_items = (int)*P.item_count;
-  const int slice0 = blockIdx.x * kNT * NS;
-  const int npass = min(NS, (N - slice0 + kNT - 1) / kNT);
-  const int total = npass * nsteps;
-  const int nchunk = (nsteps + 7) / 8;  // 1 KB DMA spans per x row
-  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)P.x, 0, (int)(uint32_t)(P.x_batch * P.M * (int64_t)K * 2), kBufFlags);
-
   for (int it_i = blockIdx.y; it_i < n_items; it_i += gridDim.y) {
     const Item it = decode_item(P, it_i);
     if (it.cnt <= 0) continue;  // block-uniform
-    const uint32_t e = __builtin_amdgcn_readfirstlane(it.expert_ok ? it.expert : 0u);
-    const bool eok = it.expert_ok;
-    if (tid < R) rowtab[tid] = item_x_row(P, it, tid);  // -1 skip, -2 NaN
+    if (threadIdx.x < 16 * MT) rowtab[threadIdx.x] = item_x_row(P, it, threadIdx.x);  // -1 skip, -2 NaN
     __syncthreads();
-    const size_t mat = (size_t)e * (uint32_t)N;
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(P.w + mat * (uint32_t)(K / 8)), 0, N * (K / 2), kBufFlags);
-    const uint16_t* const sbase = (h ? P.biases : P.scales) + mat * (uint32_t)G;
-    auto row_of = [&](int p) __attribute__((always_inline)) {
-      return (uint32_t)min(slice0 + p * kNT + 32 * wave + fr, N - 1);
-    };
-    // the epilogue of pass p: acc[i] register r is D[n = 32 wave + 8(r/4) + 4h + r%4][m = 32 i + fr]
-    // one accumulator set, k-steps in order: the ring kernel's summation order, so both
-    // instances give the same bits
-    auto store = [&](int p, const f32x16_t (&acc)[MT], bool all_nan) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = 32 * i + fr;
-        const int64_t ro = rowtab[m];
-        if (ro == -1) continue;
-        const int64_t pos = it.pos0 + m;
-        const bool nan = all_nan || ro == -2;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = slice0 + p * kNT + 32 * wave + 8 * g + 4 * h;
-          if (n >= N) continue;
-          float v[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = nan ? __builtin_nanf("") : acc[i][4 * g + q];
-          u32x2_t o;
-          o.x = pack_bf16x2(v[0], v[1]);
-          o.y = pack_bf16x2(v[2], v[3]);
-          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(P.y) + pos * N + n) = o;
-        }
-      }
-    };
-    f32x16_t acc[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-    if (!eok) {
-      for (int p = 0; p < npass; ++p) store(p, acc, true);
-      __syncthreads();
-      continue;
-    }
-    // the item's x rows: DMA span j of row r holds k-steps 8j .. 8j + 7 (lanes past the
-    // row's end or the item's rows read past x: zeros, no traffic)
-    for (int q = wave; q < R * nchunk; q += WV) {
-      const int r = q / nchunk, j = q - r * nchunk;
-      const int step = 8 * j + (lane >> 3);
-      const int c = (lane & 7) ^ ((r >> 1) & 7);
-      const int64_t ro = rowtab[r];
-      const uint32_t src = ro >= 0 && step < nsteps
-                               ? (uint32_t)ro * 2u + (uint32_t)step * 128u + 16u * c
-                               : (uint32_t)kOOB;
-      dma16(xres, smem + r * S + j * 1024, src, 0u);
-    }
-    u32x4_t wq[kXsD];
-    constexpr int kCS = kXsD / 4 + 1;  // scale/bias chunk slots: chunks in use or in flight
-    u32x2_t sbc[4];  // the chunk of steps 4c..4c+3 in slot c % 4
-    // flat step u = p * nsteps + t; nsteps % 4 == 0, so a chunk starts when u % 4 == 0
-    auto issue = [&](int u, int slot, int cslot) __attribute__((always_inline)) {
-      const int uu = min(u, total - 1);
-      const int p = uu / nsteps, t = uu - p * nsteps;
-      const uint32_t wr = row_of(p);
-      if ((u & 3) == 0)
-        sbc[cslot] = *reinterpret_cast<const u32x2_t*>(sbase + wr * (uint32_t)G + t);
-      wq[slot] = ld16(wres, wr * (uint32_t)(K / 2) + 16 * h, (uint32_t)t * 32u);
-    };
-    auto scale_bias = [&](int j, float& sc, float& bp) __attribute__((always_inline)) {
-      const u32x2_t mine = sbc[(j >> 2) & 3];
-      const uint32_t mw = (j & 2) ? mine.y : mine.x;
-      const uint32_t ow = xor32_u32(mw, lane);
-      const uint32_t sw = h ? ow : mw, bw = h ? mw : ow;
-      sc = __uint_as_float((j & 1) ? (sw & 0xFFFF0000u) : (sw << 16));
-      bp = __uint_as_float((j & 1) ? (bw & 0xFFFF0000u) : (bw << 16));
-    };
-#pragma unroll
-    for (int j = 0; j < kXsD - 1; ++j) issue(j, j, (j >> 2) & 3);
-    static_assert(kCS <= 4, "scale chunk ring");
-    // every DMA of this wave is older than the ring's loads; then all waves' rows are in
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm((kXsD - 1) + (kXsD - 2) / 4 + 1));
-    __syncthreads();
-    for (int u0 = 0; u0 < total; u0 += 16) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int u = u0 + j;
-        // step u's weights and scale chunk are in once only the younger steps' loads
-        // (u+1 .. u+kXsD-2, one each plus one per scale chunk they start) are in flight
-        const int starts = ((j + kXsD - 2) >> 2) - (j >> 2);
-        switch (starts) {
-          case 0: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXsD - 2)); break;
-          case 1: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXsD - 1)); break;
-          case 2: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXsD)); break;
-          case 3: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXsD + 1)); break;
-          default: __builtin_amdgcn_s_waitcnt(vmcnt_imm(kXsD + 2)); break;
-        }
-        if (u < total) {
-          const int p = u / nsteps, t = u - p * nsteps;
-          // the 32-row tiles that hold rows of the item (MTI = 1: rows 32..63 are padding)
-          auto compute = [&](auto mt_c) __attribute__((always_inline)) {
-            constexpr int MTI = decltype(mt_c)::value;
-            u32x4_t X[4][MTI], A[4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-              for (int i = 0; i < MTI; ++i) {
-                const int r = 32 * i + fr, c = 4 * h + ks;
-                X[ks][i] = *reinterpret_cast<const u32x4_t*>(smem + r * S + t * 128 +
-                                                             ((c ^ ((r >> 1) & 7)) << 4));
-              }
-            float sc, bp;
-            scale_bias(j, sc, bp);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) A[ks] = dequant8(wq[j % kXsD][ks], sc, bp);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-              for (int i = 0; i < MTI; ++i) acc[i] = mfma32(A[ks], X[ks][i], acc[i]);
-          };
-          compute(std::integral_constant<int, 2>{});
-          if (t == nsteps - 1) {
-            store(p, acc, false);
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-              for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-          }
-        }
-        issue(u + kXsD - 1, (j + kXsD - 1) % kXsD, ((j + kXsD - 1) >> 2) & 3);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();  // the row table and the x rows are reused by the next item
+    // (a run's rows come first: the item ends where its expert does)
+    if (MT > 2 && __builtin_amdgcn_readfirstlane((int)rowtab[8 * MT]) == -1)
+      gmm_item<MT == 2 ? 2 : MT / 2, MODE>(P, it, NS, smem, rowtab);
+    else
+      gmm_item<MT, MODE>(P, it, NS, smem, rowtab);
   }
 }
 
@@ -520,52 +358,31 @@ bool gmm_supported(int64_t N, int64_t K, int bits, int gs, int x_f32, int64_t x_
          N * (K / 2) < ((int64_t)1 << 31) && x_bytes + 2 * K < ((int64_t)1 << 31);
 }
 
-template <int MT, int WV, bool DUAL>
-hipError_t launch_mt(const QmvParams& P, int grid_items, hipStream_t s) {
-  const size_t lds = (size_t)kD * 32 * MT * 128 + 32 * MT * sizeof(int64_t);
-  static bool attr = false;
-  if (!attr) {
-    auto k = gmm_kernel<MT, WV, DUAL>;
-    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
-    if (e != hipSuccess) return e;
-    attr = true;
-  }
-  constexpr int kNT = 32 * (DUAL ? WV / 2 : WV);
-  const dim3 grid((unsigned)((P.N + kNT - 1) / kNT), (unsigned)std::max(1, grid_items));
-  hipLaunchKernelGGL((gmm_kernel<MT, WV, DUAL>), grid, dim3(64 * WV), lds, s, P);
-  return hipGetLastError();
-}
-
-bool gmm_xs_fits(int64_t K) { return (int64_t)64 * xs_row_stride((int)K) + 512 <= 160 * 1024; }
-
-hipError_t launch_gmm_xs(const QmvParams& P, int ns, int grid_items, hipStream_t s) {
-  constexpr int WV = 8, kNT = 32 * WV;
-  if (!P.items || !P.item_count || P.dual || P.swiglu_gate || !gmm_xs_fits(P.K) || ns < 1)
-    return hipErrorInvalidValue;
-  const size_t lds = (size_t)64 * xs_row_stride(P.K) + 64 * sizeof(int64_t);
-  static size_t attr = 0;
-  if (attr < lds) {
-    hipError_t e = hipFuncSetAttribute((const void*)gmm_xs_kernel<WV>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    attr = lds;
-  }
+template <int MT, int MODE>
+hipError_t launch_mt(const QmvParams& P, int ns, int grid_items, hipStream_t s) {
+  constexpr size_t lds = (size_t)kRing * 16 * MT * 128 + 16 * MT * sizeof(int64_t);
+  constexpr int kNT = 32 * (MODE == 2 ? kWaves / 2 : kWaves);
   const dim3 grid((unsigned)((P.N + kNT * ns - 1) / (kNT * ns)), (unsigned)std::max(1, grid_items));
-  hipLaunchKernelGGL(gmm_xs_kernel<WV>, grid, dim3(64 * WV), lds, s, P, ns);
+  hipLaunchKernelGGL((gmm_kernel<MT, MODE>), grid, dim3(64 * kWaves), lds, s, P, ns);
   return hipGetLastError();
 }
 
-hipError_t launch_gmm(const QmvParams& P, int mt, int grid_items, hipStream_t s) {
+hipError_t launch_gmm(const QmvParams& P, int mt, double items, int grid_items, hipStream_t s) {
   if (!P.items || !P.item_count) return hipErrorInvalidValue;
-  // 4 waves (128 weight rows) a block, three blocks a CU: 256-row blocks of 8 waves measured
-  // 233 against 216 us per configs[3] T=512 layer (two blocks a CU then)
   if (P.dual && (!P.w2 || !P.scales2 || !P.biases2)) return hipErrorInvalidValue;
-  switch (mt * 2 + (P.dual ? 1 : 0)) {
-    case 2: return launch_mt<1, 4, false>(P, grid_items, s);
-    case 3: return launch_mt<1, 4, true>(P, grid_items, s);
-    case 4: return launch_mt<2, 4, false>(P, grid_items, s);
-    case 5: return launch_mt<2, 4, true>(P, grid_items, s);
+  // passes of a block: one round of three blocks a CU, at most 64 steps a block
+  const int mode = P.dual ? 2 : P.swiglu_gate ? 1 : 0;
+  int64_t ns = 1;
+  if (mode == 0)
+    ns = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::ceil((P.N + 127) / 128 * items / 768.0),
+                                                4096 / P.K));
+  switch (mt * 4 + mode) {
+    case 4: return launch_mt<2, 0>(P, (int)ns, grid_items, s);
+    case 5: return launch_mt<2, 1>(P, 1, grid_items, s);
+    case 6: return launch_mt<2, 2>(P, 1, grid_items, s);
+    case 8: return launch_mt<4, 0>(P, (int)ns, grid_items, s);
+    case 9: return launch_mt<4, 1>(P, 1, grid_items, s);
+    case 10: return launch_mt<4, 2>(P, 1, grid_items, s);
     default: return hipErrorInvalidValue;
   }
 }

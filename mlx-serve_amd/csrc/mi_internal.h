@@ -103,11 +103,8 @@ hipError_t launch_qmvm_gather(const QmvParams& G, const QmvmPlan& plan, int grid
 // Grouped GEMM over sorted work items (gmm.hip): 4-bit affine gs 64, bf16 x; items of up to
 // 32 * mt rows (mt = 1, 2) built by launch_build_items; grid_items blocks stride them.
 bool gmm_supported(int64_t N, int64_t K, int bits, int gs, int x_f32, int64_t x_bytes);
-hipError_t launch_gmm(const QmvParams& P, int mt, int grid_items, hipStream_t s);
-// x-stationary instance for short K (the item's 64 x rows, all of K, in LDS): 64-row items,
-// ns passes of 256 weight rows a block, plain bf16 outputs only
-bool gmm_xs_fits(int64_t K);
-hipError_t launch_gmm_xs(const QmvParams& P, int ns, int grid_items, hipStream_t s);
+// items: expected work items (sizes the passes of a block)
+hipError_t launch_gmm(const QmvParams& P, int mt, double items, int grid_items, hipStream_t s);
 
 // Mid-row GEMM (midm*.hip): up to 128 rows of bf16 x. fmt: affine bits 4 or 8 (gs 64), and from
 // 33 rows 2/3/5/6 (gs 64) and 100 nvfp4, 101 mxfp4, 102 mxfp8 (uint8 scales, no biases). x and

@@ -1,0 +1,48 @@
+"""Grouped expert GEMM (sorted gather_qmm with several rows per expert) against the oracle: run
+lengths around its 16-, 32- and 64-row items, output widths that end inside a block, one step
+unit of K and several, and blocks of two passes over the output."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import BF16_TOL, max_err_ratio, to_dev_bf16, to_dev_u32, to_f64, weights
+import mi_qmm
+
+pytestmark = pytest.mark.gpu
+
+RUNS = {32: [1, 15, 16, 17, 31, 32, 33, 0], 64: [1, 31, 32, 33, 63, 64, 65, 0]}
+
+
+def _case(N, K, rows, seed):
+    runs = RUNS[rows]
+    rhs = np.repeat(np.arange(len(runs)), runs).astype(np.uint32)
+    return rhs, weights(len(runs), N, K, 4, 64, seed), O.make_x_bf16(len(rhs), K, seed + 1)
+
+
+@pytest.mark.parametrize("N,K", [(4, 256), (36, 768), (260, 2048), (12420, 256)])
+@pytest.mark.parametrize("rows", [32, 64])
+def test_runs(dev, N, K, rows):
+    print("CASE", dict(t="gmm_runs", N=N, K=K, rows=rows), flush=True)
+    rhs, (wq, s, b), x = _case(N, K, rows, N + K)
+    y = mi_qmm.gather_qmm(to_dev_bf16(x, dev).view(len(rhs), 1, K), to_dev_u32(wq, dev),
+                          to_dev_bf16(s, dev), to_dev_bf16(b, dev),
+                          rhs_indices=to_dev_u32(rhs, dev), group_size=64, bits=4,
+                          sorted_indices=True).view(len(rhs), N)
+    truth = np.concatenate([O.qmm_f64(x[rhs == e], wq[e], s[e], b[e], 64, 4)
+                            for e in range(len(wq)) if (rhs == e).any()])
+    assert max_err_ratio(to_f64(y), truth) <= BF16_TOL
+
+
+@pytest.mark.parametrize("N,K", [(4, 256), (100, 768)])
+@pytest.mark.parametrize("rows", [32, 64])
+def test_dual_matches_separate_products(dev, N, K, rows):
+    """gate + up + SwiGLU in one launch: the same products, so the same bits."""
+    rhs, (wq, s, b), x = _case(N, K, rows, 3 * N + K)
+    up = [to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev)]
+    gate = [t.flip(0).contiguous() for t in up]
+    xd, r = to_dev_bf16(x, dev).view(len(rhs), 1, K), to_dev_u32(rhs, dev)
+    kw = dict(rhs_indices=r, group_size=64, bits=4, sorted_indices=True)
+    y = mi_qmm.gather_qmm_gate_up_swiglu(xd, *gate, *up, **kw)
+    ref = mi_qmm.swiglu(mi_qmm.gather_qmm(xd, *gate, **kw), mi_qmm.gather_qmm(xd, *up, **kw))
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
