@@ -79,6 +79,28 @@ MI_DEV u32x4_t fp8_run(uint32_t w0, uint32_t w1, float sc) {
   return r;
 }
 
+// e8m0 byte 255 is infinity in the reference's reading; the conversions above give NaN for
+// every code under it. 8 codes times infinity: +-inf, or NaN for a zero code.
+template <int BITS>
+MI_DEV u32x4_t inf_run(uint32_t w0, uint32_t w1) {
+  u32x4_t r;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int c = 2 * d + i;
+      const uint32_t q = (BITS == 4 ? w0 >> (4 * c) : (c < 4 ? w0 : w1) >> (8 * (c & 3))) & ((1u << BITS) - 1u);
+      const uint32_t mag = q & ((1u << (BITS - 1)) - 1u);
+      o |= (mag ? 0x7F80u | (q >> (BITS - 1) << 15) : 0x7FC0u) << (16 * i);
+    }
+    r[d] = o;
+  }
+  return r;
+}
+// Non-zero when a byte of v is 255.
+MI_DEV uint32_t ff_bytes(uint32_t v) { return (~v - 0x01010101u) & v & 0x80808080u; }
+
 // 16 two-bit codes (LSB-first in d) -> bf16 pairs (128 + q) in natural order, codes 0..7 in
 // r0 and 8..15 in r1. Four masked shifts put codes k, k+4, k+8, k+12 in the bytes of one
 // word; v_perm pairs code 2p with code 2p+1 between zero bytes, and the OR adds the 0x43

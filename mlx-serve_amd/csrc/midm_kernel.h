@@ -29,7 +29,10 @@
 // prefill kernel's: 76 VALU a step and row tile whatever the rows, against 52 + 32 a tile.
 //
 // The bias-less modes use the 4- and 8-bit layouts; code x scale is exact in bf16
-// (code_runs.h), so they need neither epilogue nor rounding. The other widths are one
+// (code_runs.h), so they need neither epilogue nor rounding. The conversions are exact at every
+// scale byte but e8m0 255 (infinity; they give NaN): a wave that met one sums its range again
+// after the loop, straight from memory, with such groups decoded by hand (a second copy of the
+// pipelined steps spilled). The other widths are one
 // bitstream a row: a lane loads the 4 * bits bytes of its own 32 codes.
 //
 // Steps past a wave's range load through a resource of zero records (zeros, no traffic) and
@@ -174,6 +177,7 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
   constexpr bool FP = FMT >= 100;
   constexpr int BITS = fmt_bits(FMT);
   constexpr bool ODD = BITS != 4 && BITS != 8;
+  constexpr bool E8M0 = FMT == 101 || FMT == 102;
   static_assert(!EX || (!FP && !ODD), "exact codes: affine 4 and 8 bits");
   constexpr int U = 4;  // steps of a unit: the loop body, one load of scales and biases
   constexpr int CS = BITS == 4 ? 2 : 1, DC = D / CS;
@@ -302,6 +306,7 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
     return *reinterpret_cast<const u32x4_t*>(ring + (t % R) * (MT * 4096) + r * 128 +
                                              ((c ^ ((r >> 1) & 7)) << 4));
   };
+  uint32_t ff = 0;  // non-zero: a scale byte of the lane's row is 255
 #pragma unroll 1
   for (int t0 = 0; t0 < P.steps; t0 += U) {
     uint32_t sd[FMT == 100 ? 4 : 2], bd[2] = {0u, 0u};
@@ -315,6 +320,7 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
         const uint32_t mask = (g < ns ? 0xFFFFu : 0u) | (g + 1 < ns ? 0xFFFF0000u : 0u);
         sd[d] = __builtin_amdgcn_alignbit(ts[d + 1], ts[d], ssh) & mask;
         if constexpr (!FP) bd[d] = __builtin_amdgcn_alignbit(tb[d + 1], tb[d], ssh) & mask;
+        if constexpr (E8M0) ff |= code_runs::ff_bytes(sd[d]);
       }
     }
     float xs[EX ? MT : 1][U];
@@ -421,6 +427,42 @@ __global__ void __launch_bounds__(64 * WN * WK) midm_kernel(MidmParams P) {
         }
         const u32x4_t A = h ? u32x4_t{lo[0], lo[1], 0, 0} : u32x4_t{hi[0], hi[1], mi[0], mi[1]};
         acc[j] = mfma32(A, B, acc[j]);
+      }
+    }
+  }
+  if constexpr (E8M0) {
+    if (__builtin_amdgcn_ballot_w64(ff != 0u)) {
+      const __amdgpu_buffer_rsrc_t xrs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)P.x, (short)0, xrec, kBufFlags);
+      const __amdgpu_buffer_rsrc_t wrs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)P.w, (short)0, wrec, kBufFlags);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[j] = zero;
+#pragma unroll 1
+      for (int t = 0; t < ns; ++t) {
+        const uint32_t sw = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(sres, sa + 2 * t, 0, 0);
+#pragma unroll 1
+        for (int ks = 0; ks < 4; ++ks) {
+          // the 8 values that operand ks holds in the loop above
+          const int c = BITS == 4 ? 4 * h + ks : 4 * (ks / 2) + 2 * h + ks % 2;
+          const uint32_t wb = (uint32_t)min(n0 + fr, N - 1) * rowb + (uint32_t)((s0 + t) * 8 + c) * BITS;
+          const uint32_t sc = sw >> (8 * (c / 4)) & 0xFFu;  // 32-code groups
+          u32x2_t q = {0u, 0u};
+          if constexpr (BITS == 4)
+            q.x = __builtin_amdgcn_raw_buffer_load_b32(wrs, wb, 0, 0);
+          else
+            q = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(wrs, wb, 0, 0));
+          const float f = __uint_as_float(sc << 23);
+          const u32x4_t w = sc == 0xFFu ? code_runs::inf_run<BITS>(q.x, q.y)
+                            : BITS == 4 ? code_runs::fp4_run(q.x, f)
+                                        : code_runs::fp8_run(q.x, q.y, f);
+#pragma unroll
+          for (int j = 0; j < MT; ++j) {
+            const int r = 32 * j + fr;
+            const uint32_t xb = r < M ? (uint32_t)(r * K + 64 * (s0 + t) + 8 * c) * 2 : kOOB;
+            acc[j] = mfma32(__builtin_amdgcn_raw_buffer_load_b128(xrs, xb, 0, 0), w, acc[j]);
+          }
+        }
       }
     }
   }

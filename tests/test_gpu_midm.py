@@ -96,3 +96,34 @@ def test_other_formats(dev, fmt, M, N, K):
                                     torch.from_numpy(sc).to(dev), None, True, gs, bits, fmt)
         truth = O.bf16_to_f32(x).astype(np.float64) @ O.dequantize_fp(wq, sc, fmt).astype(np.float64).T
     assert max_err_ratio(to_f64(y), truth) <= BF16_TOL
+
+
+@pytest.mark.parametrize("mode", ["mxfp4", "mxfp8"])
+@pytest.mark.parametrize("M", [33, 128, 129])
+def test_scale_bytes_at_the_ends(dev, mode, M):
+    """e8m0 byte 255 is infinity (the oracle's reading): a group of non-zero codes under it gives
+    +-inf where every product has one sign and NaN where signs mix or a code is zero; bytes
+    0..7 (down to 2^-127) give their values. Other weight rows keep theirs."""
+    N, K = 36, 256
+    _, bits, gs = O.FP_MODES[mode]
+    rng = np.random.default_rng(5)
+    top = 1 << (bits - 1)  # sign bit
+    codes = rng.integers(1, top - 1, size=(N, K)).astype(np.uint8)
+    sc = np.full((N, K // gs), 120, np.uint8)
+    sc[0, 1] = sc[1, 7] = sc[2, 3] = sc[3, 4] = sc[35, 7] = 255
+    codes[1] |= top               # -inf
+    codes[2, 3 * gs + 5] = 0      # zero times infinity
+    codes[3, 4 * gs + 9] |= top   # mixed signs
+    sc[8:16] = np.arange(8)[:, None]
+    x = np.abs(O.bf16_to_f32(O.make_x_bf16(M, K, 6))) + 0.5
+    x = O.f32_to_bf16(x * np.float32(2.0 ** 30))
+    y = to_f64(mi_qmm.quantized_matmul(to_dev_bf16(x, dev), to_dev_u32(O.pack(codes, bits), dev),
+                                       torch.from_numpy(sc).to(dev), None, True, gs, bits, mode))
+    with np.errstate(invalid="ignore"):
+        w = O.dequantize_fp(O.pack(codes, bits), sc, mode).astype(np.float64)
+        truth = O.bf16_to_f32(x).astype(np.float64) @ w.T
+    assert np.isposinf(truth[:, [0, 35]]).all() and np.isneginf(truth[:, 1]).all()
+    assert np.isnan(truth[:, 2:4]).all()
+    np.testing.assert_array_equal(y[:, [0, 1, 2, 3, 35]], truth[:, [0, 1, 2, 3, 35]])
+    for n in range(4, 35):  # per output column: the scales differ by orders of magnitude
+        assert max_err_ratio(y[:, n:n + 1], truth[:, n:n + 1]) <= BF16_TOL, n
