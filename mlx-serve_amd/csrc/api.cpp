@@ -997,23 +997,28 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   static const int use_dqgemm = env_int("MI_QMM_DQGEMM", 0);
   static const int prefill_min = env_int("MI_QMM_PREFILL_MIN", 128);
   // 17..128 rows at gs 64: the mid-row kernel. Up to 32 rows only where a 32-row launch of the
-  // few-row kernel fills the GPU at 8 weight tiles a block and this kernel's blocks are wide
-  // (4-bit [14336,4096] 32 rows 19.3 -> 15.9 us, [4096,14336] 19.0 -> 18.2; elsewhere level or
-  // behind: 8-bit [2048,7168] 10.8 against 11.2, 4-bit [2048,768] 4.7 against 5.3). On those
-  // shapes 33..48 rows run as 32 rows here and the rest on the few-row kernel, so that every
-  // row keeps the bits of the separate calls (30.3 -> 26.9 us at 48 rows; one launch 21.3);
-  // from 49 rows on this kernel alone has them (37.5 -> 21.7 us at 64 rows).
+  // few-row kernel fills the GPU at 8 weight tiles a block (4-bit [14336,4096] 32 rows 19.3 ->
+  // 15.9 us, [4096,14336] 19.0 -> 18.2; elsewhere level or behind: 8-bit [2048,7168] 10.8 against
+  // 11.2, 4-bit [2048,768] 4.7 against 5.3). On those shapes 33..48 rows run as 32 rows here and
+  // the rest on the few-row kernel, so that every row keeps the bits of the separate calls (30.3
+  // -> 26.9 us at 48 rows; one launch 21.3); from 49 rows on this kernel alone has them (37.5 ->
+  // 21.7 us at 64 rows). Whether a shape is one of them must not depend on M either, so the few
+  // where this kernel is behind at 17..32 rows stay with it: 8-bit [5888,11264] 17 rows 24.1 ->
+  // 28.4 us, 32 rows 26.0 -> 29.8, against [4608,8192] 32 rows 22.7 -> 18.9, [6656,2560] 14.5 ->
+  // 8.4, 4-bit [5120,5120] 0.85 of the few-row kernel's time.
   static const int use_midm = env_int("MI_QMM_MIDM", 1);
   mi::MidmPlan mp{};
   if (use_midm && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 && (nb == 4 || nb == 8) &&
-      midm_aligned(x, w, scales, biases, y) && mi::midm_plan(M, N, K, nb, gs, &mp) &&
-      (M > 32 || (mp.wide && few_row_fills(N, K, gs, nb)))) {
-    const int64_t rows = M > 32 && M <= 48 && mp.wide && few_row_fills(N, K, gs, nb) ? 32 : M;
-    rc = run_midm(x, w, scales, biases, y, rows, N, K, nb, mp, s);
-    if (rc || rows == M) return rc;
-    return mi_quantized_matmul((uint16_t*)y + rows * N, (const uint16_t*)x + rows * K, w, scales,
-                               biases, M - rows, N, K, transpose, group_size, bits, mode, x_dtype,
-                               sb_dtype, stream);
+      midm_aligned(x, w, scales, biases, y) && mi::midm_plan(M, N, K, nb, gs, &mp)) {
+    const bool fills = M <= 48 && few_row_fills(N, K, gs, nb);
+    if (M > 32 || fills) {
+      const int64_t rows = fills && M > 32 ? 32 : M;
+      rc = run_midm(x, w, scales, biases, y, rows, N, K, nb, mp, s);
+      if (rc || rows == M) return rc;
+      return mi_quantized_matmul((uint16_t*)y + rows * N, (const uint16_t*)x + rows * K, w, scales,
+                                 biases, M - rows, N, K, transpose, group_size, bits, mode,
+                                 x_dtype, sb_dtype, stream);
+    }
   }
   if (x_dtype == MI_DTYPE_BFLOAT16 && !use_dqgemm && M >= prefill_min &&
       mi::prefill_supported(M, N, K, nb, gs)) {

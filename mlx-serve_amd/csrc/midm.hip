@@ -21,30 +21,30 @@ bool midm_plan(int64_t M, int64_t N, int64_t K, int fmt, int gs, MidmPlan* out) 
   const int bits = midm::fmt_bits(fmt);
   const bool ex = fmt == 4 || fmt == 8;
   // affine groups of 64 (a bias-less mode has its own), 4-output stores, 32-bit offsets
-  if ((fmt < 100 && gs != 64) || M < (ex ? 1 : 33) || M > 128 || N < 4 || N % 4 || K % 64 ||
+  if ((fmt < 100 && gs != 64) || M < (ex ? 17 : 33) || M > 128 || N < 4 || N % 4 || K % 64 ||
       M * K * 2 >= ((int64_t)1 << 31) || N * (K * bits / 8) >= ((int64_t)1 << 31) ||
       N >= ((int64_t)1 << 30))
     return false;
-  // Block shape (64 rows x 4 K parts, or 32 rows x 8 or 4 parts) and K split by estimated
+  // Block shape (64 or 32 rows, 4 K parts) and K split by estimated
   // time: rounds of 256 blocks x (3.6 us + steps of a wave x the time of a step), plus 3 us
   // for the partials and their reduce launch when K splits over blocks. A step costs the
   // larger of its compute (measured on half-empty grids) and its bytes from L2 at the rate
   // of a full grid. Estimates against measured at 4 bits, us: [14336,4096] 32 rows 14.8 /
-  // 15.8, 128 rows 24.9 / 27.5 (wide); [7168,2048] 32 rows 6.6 / 7.0, 128 rows 12.4 / 10.9
-  // (narrow; wide measured 8.3 and 13.7); [4096,14336] 32 rows 17.8 / 18.4 (wide, 4 ranges;
+  // 15.8, 128 rows 24.9 / 27.5 (wide); [7168,2048] 64 rows 9.2 / 9.2, 128 rows 12.4 / 10.9
+  // (narrow; wide measured 13.7 at 128); [4096,14336] 32 rows 17.8 / 18.4 (wide, 4 ranges;
   // narrow 21.7).
   // Up to 64 rows the choice does not look at M, so a row's result does not depend on how
-  // many rows ride along (wide blocks: same K parts, same order).
+  // many rows ride along (same K parts, same order).
   const int64_t rows = M <= 64 ? 32 : M;
   const int mt = (int)((rows + 31) / 32);
   static constexpr double kStep[2][4] = {{0.70, 0.65, 0.65, 0.80}, {0.70, 0.80, 0.95, 1.10}};
   const int64_t groups = K / 64;
   double best = 1e30;
   for (int wide = 0; wide < 2; ++wide) {
-    const int wk = wide || M > 32 ? 4 : 8;
+    constexpr int wk = 4;
     const int64_t tiles = (N + (wide ? 63 : 31)) / (wide ? 64 : 32);
     const double kb = (wide ? 2 : 1) * wk * 1.15 * bits / 4 + wk * rows * 0.128;
-    const double rate = wide ? 50.0 : wk == 8 ? 45.0 : 75.0;  // KB/us of a block, grid full
+    const double rate = wide ? 50.0 : 75.0;  // KB/us of a block, grid full
     for (int64_t ks = 1; ks == 1 || (tiles * ks <= 256 && ks <= 32); ++ks) {
       const int64_t steps = (groups + wk * ks * 2 - 1) / (wk * ks * 2) * 2;
       if ((groups + wk * steps - 1) / (wk * steps) != ks) continue;  // a range without steps

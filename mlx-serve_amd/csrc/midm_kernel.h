@@ -518,7 +518,7 @@ hipError_t launch_fmt(const MidmParams& P, bool wide, hipStream_t s) {
   const int mt = (P.M + 31) / 32;
   if constexpr (EX)
     if (mt == 1)
-      return wide ? launch_one<FMT, true, 1, 2, 4, 4>(P, s) : launch_one<FMT, true, 1, 1, 8, 4>(P, s);
+      return wide ? launch_one<FMT, true, 1, 2, 4, 4>(P, s) : launch_one<FMT, true, 1, 1, 4, 4>(P, s);
   if (wide)
     return mt <= 2   ? launch_one<FMT, EX, 2, 2, 4, 4>(P, s)
            : mt == 3 ? launch_one<FMT, false, 3, 2, 4, 2>(P, s)

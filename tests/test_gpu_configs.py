@@ -87,6 +87,22 @@ def test_config1_decode_sweep(dev, N, K, name, bits):
         assert err <= BF16_TOL, (M, err)
 
 
+@pytest.mark.parametrize("N,K,bits", [(5120, 5120, 4), (5120, 5120, 8), (6144, 4096, 8),
+                                      (5632, 2560, 8), (1536, 11776, 4)])
+def test_wide_rows_keep_the_bits_of_separate_calls(dev, N, K, bits):
+    """As above on other shapes whose 32-row launch fills the GPU, where the block shape that is
+    best for 32 rows alone is another than for 64."""
+    W = dev_weight(dev, N, K, bits, seed(2, 1, 40 + bits))
+    x = dev_x(dev, 64, K, seed(2, 0, 41 + bits))
+    bits_of = lambda t: t.view(torch.int16)
+    for M in (40, 48, 64):
+        _case(t="wide_rows", N=N, K=K, bits=bits, M=M)
+        y = mi_qmm.quantized_matmul(x[:M].contiguous(), *W, True, 64, bits)
+        a = mi_qmm.quantized_matmul(x[:32].contiguous(), *W, True, 64, bits)
+        b = mi_qmm.quantized_matmul(x[32:M].contiguous(), *W, True, 64, bits)
+        assert torch.equal(bits_of(y), torch.cat([bits_of(a), bits_of(b)])), M
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("N,K", [(14336, 4096), (4096, 14336)])
 def test_config1_decode_33_to_64_rows(dev, N, K, bits):

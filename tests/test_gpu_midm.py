@@ -38,6 +38,27 @@ def test_rows_and_tails(dev, M, N, K, bits):
         assert np.linalg.norm(err) <= 2.0 ** -9 * 1.01 * np.linalg.norm(truth)
 
 
+# Wide enough that 17..32 rows take this kernel (one 32-row tile): widths that end inside a block
+# of 64 rows, K ranges that end inside a wave's steps, K splits over blocks, and (2560) blocks of
+# 32 rows.
+@pytest.mark.parametrize("N,K,bits", [(14340, 4224, 4), (14340, 4224, 8), (5124, 5120, 4),
+                                      (4100, 14336, 8), (6148, 2560, 8)])
+def test_few_rows_of_wide_shapes(dev, N, K, bits):
+    G, rng = K // 64, np.random.default_rng(N + bits)
+    wq = rng.integers(0, 1 << 32, size=(N, K * bits // 32), dtype=np.uint32)
+    s = O.f32_to_bf16(rng.uniform(0.5, 1.5, size=(N, G)).astype(np.float32) / 2 ** bits)
+    b = O.f32_to_bf16(rng.uniform(-0.6, -0.4, size=(N, G)).astype(np.float32))
+    x = O.make_x_bf16(48, K, N)
+    cols = np.unique(np.concatenate([np.arange(40), rng.integers(0, N, 60), np.arange(N - 70, N)]))
+    truth = O.qmm_f64(x, wq[cols], s[cols], b[cols], 64, bits)
+    X, W, S, B = to_dev_bf16(x, dev), to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev)
+    for M in (17, 31, 32, 33, 48):
+        print("CASE", dict(t="midm_few", M=M, N=N, K=K, bits=bits), flush=True)
+        y = to_f64(mi_qmm.quantized_matmul(X[:M].contiguous(), W, S, B, True, 64, bits)[:, cols])
+        # one bf16 rounding of the result, as above
+        assert np.linalg.norm(y - truth[:M]) <= 2.0 ** -9 * 1.01 * np.linalg.norm(truth[:M])
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_rows_are_independent(dev, bits):
     """Infinite and NaN activations stay in their rows, and scales of the next weight row (read
