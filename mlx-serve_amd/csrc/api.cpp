@@ -275,7 +275,7 @@ struct GatherJob {
   bool empty = false, narrow = false, use_items = false, one_row = false, multi_row = false;
   bool grouped = false;  // sorted runs on the grouped kernel (gmm.hip)
   int gmm_mt = 0;        // its 32-row tiles per item
-  double gmm_items = 0;  // expected work items (distinct experts x items per run)
+  double gmm_items = 0;  // expected work items (distinct experts x items of a run)
   int64_t max_items = 0;
   size_t items_bytes = 0, part_bytes = 0;
   size_t items_region() const { return ((items_bytes + 255) / 256) * 256; }
@@ -362,10 +362,16 @@ int gather_prepare(GatherJob& J, void* y, const void* x, const uint32_t* w, cons
       if (mu >= gmm_min) {
         const double want = mu + 3.0 * std::sqrt(mu);
         J.grouped = true;
-        J.gmm_items = distinct * std::max(1.0, std::ceil(want / 64.0));
         static const int force_mt = env_int("MI_QMM_GMM_MT", 0);
         J.gmm_mt = force_mt == 1 || force_mt == 2 ? force_mt
                    : want <= 32 ? 1 : 2;  // longer runs are cut into 64-row items
+        // expected items: a run of X rows, about normal with mean and variance mu, is cut into
+        // ceil(X / item rows)
+        const double rpi = 32.0 * J.gmm_mt;
+        double per = mu > 8.0 * rpi ? mu / rpi + 0.5 : 1.0;
+        for (int j = 1; mu <= 8.0 * rpi && j <= 16; ++j)
+          per += 0.5 * std::erfc((rpi * j + 0.5 - mu) / std::sqrt(2.0 * mu));
+        J.gmm_items = distinct * per;
       }
     }
     J.narrow = q16 && avg <= 4;

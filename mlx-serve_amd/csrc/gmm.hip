@@ -24,14 +24,13 @@
 // One barrier a step, before its second k-step, whose MFMAs carry the LDS reads of the next
 // step's first fragments; every MFMA group carries half of the next step's dequantize. Vector
 // memory operations return in order, so "x stage t + 1 has arrived" is an exact vmcnt. A block
-// with several passes (short K) runs them as one stream of steps, so the rings never drain.
+// with two passes runs them as one stream of steps, so the rings never drain.
 //
 // Measured, us a call, 4 bits, before -> after: gate + up of 128 experts [768,2048], top 8, 64
 // tokens 84.5 -> 74.6, 512 tokens 100 -> 90; 256 experts [2048,7168], 512 tokens 1765 -> 1471;
-// down projections [2048,768] 64 tokens 42.9 -> 37.9, 512 tokens 52.5 -> 54.4 (64 x rows held
-// in LDS then), [2048,1536] (64 experts, top 6) 512 tokens 61 -> 56, [7168,2048] 690 -> 602.
+// down projections [2048,768] 64 tokens 42.9 -> 37.9, 600 tokens 51.9 -> 51.6 (64 x rows held in
+// LDS then), [2048,1536] (64 experts, top 6) 500 tokens 58 -> 50, [7168,2048] 690 -> 602.
 #include <algorithm>
-#include <cmath>
 
 #include "dequant_bf16.h"
 #include "mi_common.h"
@@ -370,17 +369,21 @@ hipError_t launch_mt(const QmvParams& P, int ns, int grid_items, hipStream_t s) 
 hipError_t launch_gmm(const QmvParams& P, int mt, double items, int grid_items, hipStream_t s) {
   if (!P.items || !P.item_count) return hipErrorInvalidValue;
   if (P.dual && (!P.w2 || !P.scales2 || !P.biases2)) return hipErrorInvalidValue;
-  // passes of a block: one round of three blocks a CU, at most 64 steps a block
   const int mode = P.dual ? 2 : P.swiglu_gate ? 1 : 0;
-  int64_t ns = 1;
-  if (mode == 0)
-    ns = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::ceil((P.N + 127) / 128 * items / 768.0),
-                                                4096 / P.K));
+  // Passes of a block: one, since more blocks than a round (three a CU) even out items of
+  // different rows. us a call, as many passes as one round takes (2 or 3) -> 1: [2048,768] of 128
+  // experts, 500 tokens 52.9 -> 47.3, 900 tokens 87.0 -> 61.1; [2048,1536] of 64, 600 tokens 69.3
+  // -> 54.6; [1536,2048] of 64, 500 tokens 51.9 -> 46.2. Two where one leaves a second round with
+  // few blocks: [1536,2048] of 64 experts, 600 tokens (1.14 rounds) 59.0 -> 54.7, of K = 1024 39.3
+  // -> 37.9, 4096 123 -> 106; [768,2048] of 128, 950 tokens (1.25) 67.3 -> 61.1. At 1.33 rounds one
+  // pass is ahead again ([2048,1536] of 64, 450 tokens 47.2 against 52.6; 1.74 rounds 10-30%).
+  const double rounds = (double)((P.N + 127) / 128) * items / 768.0;
+  const int ns = mode == 0 && rounds > 1.03 && rounds < 1.33 ? 2 : 1;
   switch (mt * 4 + mode) {
-    case 4: return launch_mt<2, 0>(P, (int)ns, grid_items, s);
+    case 4: return launch_mt<2, 0>(P, ns, grid_items, s);
     case 5: return launch_mt<2, 1>(P, 1, grid_items, s);
     case 6: return launch_mt<2, 2>(P, 1, grid_items, s);
-    case 8: return launch_mt<4, 0>(P, (int)ns, grid_items, s);
+    case 8: return launch_mt<4, 0>(P, ns, grid_items, s);
     case 9: return launch_mt<4, 1>(P, 1, grid_items, s);
     case 10: return launch_mt<4, 2>(P, 1, grid_items, s);
     default: return hipErrorInvalidValue;

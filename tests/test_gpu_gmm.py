@@ -46,3 +46,21 @@ def test_dual_matches_separate_products(dev, N, K, rows):
     y = mi_qmm.gather_qmm_gate_up_swiglu(xd, *gate, *up, **kw)
     ref = mi_qmm.swiglu(mi_qmm.gather_qmm(xd, *gate, **kw), mi_qmm.gather_qmm(xd, *up, **kw))
     assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+def test_two_passes_a_block(dev):
+    """A count of blocks a little over a round (three a CU), where a block makes two passes over
+    the output: 235 tiles of 128 rows x about 3.7 items of one expert; the last block has one pass
+    that ends inside a tile."""
+    N, K, T = 30020, 512, 200
+    rng = np.random.default_rng(3)
+    wq = rng.integers(0, 1 << 32, size=(1, N, K // 8), dtype=np.uint32)
+    s = O.f32_to_bf16(rng.uniform(0.05, 0.1, size=(1, N, K // 64)).astype(np.float32))
+    b = O.f32_to_bf16(rng.uniform(-0.6, -0.4, size=(1, N, K // 64)).astype(np.float32))
+    x, rhs = O.make_x_bf16(T, K, 4), np.zeros(T, np.uint32)
+    y = mi_qmm.gather_qmm(to_dev_bf16(x, dev).view(T, 1, K), to_dev_u32(wq, dev), to_dev_bf16(s, dev),
+                          to_dev_bf16(b, dev), rhs_indices=to_dev_u32(rhs, dev), group_size=64,
+                          bits=4, sorted_indices=True).view(T, N)
+    cols = np.unique(np.concatenate([np.arange(260), rng.integers(0, N, 300), np.arange(N - 300, N)]))
+    truth = O.qmm_f64(x, wq[0][cols], s[0][cols], b[0][cols], 64, 4)
+    assert max_err_ratio(to_f64(y[:, cols]), truth) <= BF16_TOL
