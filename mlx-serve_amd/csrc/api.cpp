@@ -351,7 +351,7 @@ int gather_prepare(GatherJob& J, void* y, const void* x, const uint32_t* w, cons
     if (item_rows > 0) avg = item_rows;
     // Runs that average several rows per distinct expert go to the grouped kernel: one
     // block per (item, 128-row weight tile) streams the tile once for all the item's rows
-    // (up to 32 * MT), in-register dequantize into 32x32x16 MFMAs. Items are sized for
+    // (up to 32 * MT), in-register dequantize into 16x16x32 MFMAs. Items are sized for
     // mu + 3 sigma rows as above, so a run is rarely cut.
     static const int use_gmm = env_int("MI_QMM_GMM", 1);
     static const int gmm_min = env_int("MI_QMM_GMM_MIN_ROWS", 4);
@@ -964,7 +964,7 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
     }
     // 33..128 rows: the mid-row kernel, against dequantize + the bf16 GEMM (mxfp4 [14336,4096]
     // 64 rows 123 -> 17 us, 128 rows 129 -> 26; mxfp8 136 -> 25, 140 -> 33)
-    static const int fp_midm = env_int("MI_QMM_MIDM", 1);
+    static const int fp_midm = env_int("MI_QMM_MIDM", 1) && !env_int("MI_QMM_DQGEMM", 0);
     mi::MidmPlan mp{};
     if (fp_midm && M > 32 && M <= 128 && midm_aligned(x, w, scales, nullptr, y) &&
         mi::midm_plan(M, N, K, 100 + fm, gs, &mp))
@@ -990,15 +990,20 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   if (N > (int64_t)1 << 30 || M > (int64_t)1 << 30) return fail(MI_ERR_INVALID, "N or M too large");
   hipStream_t s = (hipStream_t)stream;
   // Dispatch, in order:
-  //  - 4- and 8-bit weights at M >= MI_QMM_PREFILL_MIN (default 128): the fused prefill kernel
-  //    (prefill.hip), which replaces the reference's prefillDqGemm route
-  //    (src/transformer.zig:20987-21011) without a bf16 copy of the weight;
+  //  - 4- and 8-bit weights at gs 64: the mid-row kernel (midm_kernel.h) at 33..128 rows, and at
+  //    17..32 on wide shapes; MI_QMM_MIDM=0 turns it off for every format;
+  //  - 4- and 8-bit weights at M >= MI_QMM_PREFILL_MIN (default 128, which leaves gs 64 to the
+  //    mid-row kernel up to 128 rows; a value that is set applies to gs 64 as well): the fused
+  //    prefill kernels (prefill.hip, prefill128.hip), which replace the reference's
+  //    prefillDqGemm route (src/transformer.zig:20987-21011) without a bf16 copy of the weight;
   //  - one row of gs-64 2/3/5/6/8-bit weights: the one-row streaming kernel;
-  //  - 2/3/5/6 bits: the few-row MFMA kernel (2..32 rows, gs 64), qmv_any (up to
-  //    MI_QMM_ANY_MAX rows), else dequantize to bf16 + the prefill kernel's bf16 instance;
-  //  - 4/8 bits: the few-row MFMA kernel (up to 64 rows), else the fused qmm kernel.
-  //    Dequantize + hipBLASLt is opt-in for every format (MI_QMM_DQGEMM=1; for 4/8 bits from
-  //    MI_QMM_DQGEMM_MIN rows).
+  //  - 2/3/5/6 bits: the few-row MFMA kernel (2..32 rows, gs 64), the mid-row kernel (33..128,
+  //    gs 64), qmv_any (up to MI_QMM_ANY_MAX rows), else dequantize to bf16 + the prefill
+  //    kernels' bf16 instances;
+  //  - 4/8 bits: the few-row MFMA kernel (up to 64 rows; above 16 or 32 only layouts that the
+  //    mid-row kernel declines, as N % 4 != 0 and unaligned pointers), else the fused qmm kernel.
+  //    Dequantize + hipBLASLt is opt-in for every format (MI_QMM_DQGEMM=1; 2/3/5/6 bits and
+  //    the fp modes above the few-row kernel's 32 rows, 4/8 bits from MI_QMM_DQGEMM_MIN rows).
   static const int dq_min = env_int("MI_QMM_DQGEMM_MIN", 256);
   static const int use_dqgemm = env_int("MI_QMM_DQGEMM", 0);
   static const int prefill_min = env_int("MI_QMM_PREFILL_MIN", 128);
@@ -1012,10 +1017,14 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   // where this kernel is behind at 17..32 rows stay with it: 8-bit [5888,11264] 17 rows 24.1 ->
   // 28.4 us, 32 rows 26.0 -> 29.8, against [4608,8192] 32 rows 22.7 -> 18.9, [6656,2560] 14.5 ->
   // 8.4, 4-bit [5120,5120] 0.85 of the few-row kernel's time.
+  // (rows that MI_QMM_PREFILL_MIN or MI_QMM_DQGEMM ask for another route keep it)
   static const int use_midm = env_int("MI_QMM_MIDM", 1);
+  static const bool prefill_set = getenv("MI_QMM_PREFILL_MIN") != nullptr;
+  const bool other_route = (prefill_set && M >= prefill_min) || (use_dqgemm && dq_min > 0 && M >= dq_min);
   mi::MidmPlan mp{};
-  if (use_midm && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 && (nb == 4 || nb == 8) &&
-      midm_aligned(x, w, scales, biases, y) && mi::midm_plan(M, N, K, nb, gs, &mp)) {
+  if (use_midm && !other_route && x_dtype == MI_DTYPE_BFLOAT16 && M >= 17 && M <= 128 &&
+      (nb == 4 || nb == 8) && midm_aligned(x, w, scales, biases, y) &&
+      mi::midm_plan(M, N, K, nb, gs, &mp)) {
     const bool fills = M <= 48 && few_row_fills(N, K, gs, nb);
     if (M > 32 || fills) {
       const int64_t rows = fills && M > 32 ? 32 : M;
@@ -1104,8 +1113,8 @@ int mi_quantized_matmul(void* y, const void* x, const uint32_t* w, const void* s
   }
   // 33..128 rows: the mid-row kernel, against dequantize + the bf16 GEMM (6-bit [14336,4096] 64
   // rows 129 -> 45 us, 128 rows 135 -> 52; 2-bit 110 -> 20, 116 -> 28)
-  if (use_midm && odd_width && M > 32 && M <= 128 && midm_aligned(x, w, scales, biases, y) &&
-      mi::midm_plan(M, N, K, nb, gs, &mp))
+  if (use_midm && !use_dqgemm && odd_width && M > 32 && M <= 128 &&
+      midm_aligned(x, w, scales, biases, y) && mi::midm_plan(M, N, K, nb, gs, &mp))
     return run_midm(x, w, scales, biases, y, M, N, K, nb, mp, s);
   static const int any_max = env_int("MI_QMM_ANY_MAX", 8);
   if (odd_width && M <= any_max) {  // decode rows: straight from the packed bitstream
