@@ -106,9 +106,9 @@ def test_wide_rows_keep_the_bits_of_separate_calls(dev, N, K, bits):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("N,K", [(14336, 4096), (4096, 14336)])
 def test_config1_decode_33_to_64_rows(dev, N, K, bits):
-    """33..64 rows at the Llama-3-8B MLP shapes run as a 32-row launch plus one for the rest:
-    bit-equal to those two calls made separately, and sampled rows (both sides of the cut)
-    against the oracle."""
+    """33..64 rows at the Llama-3-8B MLP shapes (up to 48 a 32-row launch of the mid-row kernel and
+    a few-row one, above one mid-row launch): bit-equal to a 32-row call and one for the rest made
+    separately, and sampled rows (both sides of the cut) against the oracle."""
     W = dev_weight(dev, N, K, bits, seed(2, 1, 9 + bits))
     x = dev_x(dev, 64, K, seed(2, 0, 5 + bits))
     for M in (33, 48, 64):

@@ -64,3 +64,20 @@ def test_two_passes_a_block(dev):
     cols = np.unique(np.concatenate([np.arange(260), rng.integers(0, N, 300), np.arange(N - 300, N)]))
     truth = O.qmm_f64(x, wq[0][cols], s[0][cols], b[0][cols], 64, 4)
     assert max_err_ratio(to_f64(y[:, cols]), truth) <= BF16_TOL
+
+
+def test_scales_on_an_odd_half(dev):
+    """Banks whose scales and biases start on an odd half: the same bits as aligned ones."""
+    rhs, (wq, s, b), x = _case(100, 768, 64, 11)
+
+    def off(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)
+        v = buf[1:].view(t.shape)
+        v.copy_(t)
+        return v
+    xd, r = to_dev_bf16(x, dev).view(len(rhs), 1, 768), to_dev_u32(rhs, dev)
+    W, S, B = to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev)
+    kw = dict(rhs_indices=r, group_size=64, bits=4, sorted_indices=True)
+    ref = mi_qmm.gather_qmm(xd, W, S, B, **kw)
+    y = mi_qmm.gather_qmm(xd, W, off(S), off(B), **kw)
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))

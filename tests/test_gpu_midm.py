@@ -1,7 +1,7 @@
-"""The mid-row kernel (17..128 rows, affine 4- and 8-bit, groups of 64) against the oracle where
-its tiling can go wrong: row counts around each 32-row tile, output widths that end inside a
-block, K ranges that do not divide into the waves' steps (odd group counts, so a row's scales
-start in the middle of a dword), and splits over blocks."""
+"""The mid-row kernel (33..128 rows, and 17..32 on wide shapes) against the oracle where its tiling
+can go wrong: row counts around each 32-row tile, output widths that end inside a block, K ranges
+that do not divide into the waves' steps (odd group counts, so a row's scales start in the middle of
+a dword), and splits over blocks; and the layouts beside it that take other kernels."""
 import numpy as np
 import pytest
 import torch
@@ -27,14 +27,16 @@ def _run(dev, M, N, K, bits, seed):
 @pytest.mark.parametrize("N,K", SHAPES)
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
 def test_rows_and_tails(dev, M, N, K, bits):
+    """(17 and 32 rows of these narrow shapes run on the few-row kernel, with the same bound.)"""
     print("CASE", dict(t="midm", M=M, N=N, K=K, bits=bits), flush=True)
     x, w, y = _run(dev, M, N, K, bits, 100 * M + N)
     truth = O.qmm_f64(x, *w, 64, bits)
     err = to_f64(y) - truth
     assert max_err_ratio(to_f64(y), truth) <= BF16_TOL
     if M <= 64:
-        # exact codes and fp32 sums: what is left is one bf16 rounding of the result, at most
-        # 2^-9 of a value (2-norm below 2^-9 in all), and fp32 sums 1000 times smaller
+        # exact codes and fp32 sums: what is left is one bf16 rounding of the result, half of 2^-7
+        # of its binade at most (uniform: 2^-7 / sqrt(12), over values spread evenly on a log scale
+        # 1.5e-3 in the 2-norm, below 2^-9), and fp32 sums 1000 times smaller
         assert np.linalg.norm(err) <= 2.0 ** -9 * 1.01 * np.linalg.norm(truth)
 
 
@@ -81,7 +83,7 @@ def test_rows_are_independent(dev, bits):
 
 
 def test_unaligned_pointers_take_another_route(dev):
-    """Views that start off a 16-byte (x, w) or dword (scales) boundary still give the result."""
+    """Views that start off a 16-byte (x, w) or dword (scales, biases) boundary still give the result."""
     M, N, K = 48, 128, 512
     x, (wq, s, b), y = _run(dev, M, N, K, 4, 77)
 
@@ -92,8 +94,29 @@ def test_unaligned_pointers_take_another_route(dev):
         return v
     X, W, S, B = (to_dev_bf16(x, dev), to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev))
     truth = O.qmm_f64(x, wq, s, b, 64, 4)
-    for args in ((off(X, 4), W, S, B), (X, off(W, 1), S, B)):
+    for args in ((off(X, 4), W, S, B), (X, off(W, 1), S, B), (X, W, off(S, 1), B), (X, W, S, off(B, 1))):
         assert max_err_ratio(to_f64(mi_qmm.quantized_matmul(*args, True, 64, 4)), truth) <= BF16_TOL
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_widths_off_four_columns(dev, bits):
+    """33..64 rows of a wide output that is no multiple of 4 columns: two launches of the few-row
+    kernel, with the bits of the separate calls."""
+    N, K = 24578, 512
+    rng = np.random.default_rng(bits)
+    wq = rng.integers(0, 1 << 32, size=(N, K * bits // 32), dtype=np.uint32)
+    s = O.f32_to_bf16(rng.uniform(0.5, 1.5, size=(N, K // 64)).astype(np.float32) / 2 ** bits)
+    b = O.f32_to_bf16(rng.uniform(-0.6, -0.4, size=(N, K // 64)).astype(np.float32))
+    x = O.make_x_bf16(64, K, 7)
+    X, w = to_dev_bf16(x, dev), (to_dev_u32(wq, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev))
+    mm = lambda t: mi_qmm.quantized_matmul(t.contiguous(), *w, True, 64, bits)
+    cols = np.concatenate([np.arange(130), np.arange(N - 130, N)])
+    truth = O.qmm_f64(x, wq[cols], s[cols], b[cols], 64, bits)
+    for M in (34, 48, 64):
+        print("CASE", dict(t="off_four", M=M, bits=bits), flush=True)
+        y = mm(X[:M])
+        assert torch.equal(y.view(torch.int16), torch.cat([mm(X[:32]), mm(X[32:M])]).view(torch.int16))
+        assert max_err_ratio(to_f64(y[:, cols]), truth[:M]) <= BF16_TOL
 
 
 @pytest.mark.parametrize("fmt", [2, 3, 5, 6, "nvfp4", "mxfp4", "mxfp8"])

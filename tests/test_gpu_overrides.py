@@ -47,10 +47,9 @@ def test_vendor_gemm_on_request(dev):
 
 
 def test_prefill_from_fewer_rows(dev):
-    """MI_QMM_PREFILL_MIN=64: the prefill kernel, which rounds the weights to bf16. The exact
-    codes of the default route leave the output's rounding alone, 2^-9 of a value at most and
-    uniform below that: 2^-9 / sqrt(3) times the mean ratio of a value to its binade's top
-    (0.72), 0.8e-3; rounded weights add as much again (independent: times sqrt(2))."""
+    """MI_QMM_PREFILL_MIN=64: the prefill kernel, which rounds the weights to bf16. The exact codes
+    of the default route leave one rounding of the output (half of 2^-7 of its binade, about 1.6e-3
+    in the 2-norm); rounded weights add an independent error of the same size (times sqrt(2))."""
     exact, _ = _err(dev, 64, 4)
     err, calls = _under({"MI_QMM_PREFILL_MIN": "64"}, 64, 4)
     assert calls == 0 and 1.2 * exact < err < 5e-3

@@ -380,7 +380,8 @@ PREFILL_CASES = [(33, 64, 256), (128, 256, 512), (257, 300, 1024), (512, 520, 20
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("M,N,K", PREFILL_CASES)
 def test_prefill_qmm(dev, M, N, K, bits, gs):
-    """Large-M paths: the fused MFMA GEMM (M < 256) and dequantize + hipBLASLt (M >= 256)."""
+    """Large-M paths: the mid-row kernel (33..128 rows at gs 64), the fused MFMA GEMM (33..127 rows
+    otherwise) and the prefill kernels (above)."""
     _print_case(t="prefill", M=M, N=N, K=K, bits=bits, gs=gs)
     wq, s, b = weights(1, N, K, bits, gs, 5000 + M)
     x = O.make_x_bf16(M, K, 6000 + N)
