@@ -9,7 +9,7 @@
 // item's rows.
 //
 // What bounds it: the weight stream (226 MB a gate + up call of 128 experts, [768,2048]) as far
-// as the arithmetic keeps up: 3.0 TB/s, where a read of the same pieces alone reaches 5.8. When
+// as the arithmetic keeps up: 3.0 TB/s, where a timing build with the loads alone reached 5.8. When
 // each wave ran barrier, LDS reads, MFMAs and dequantize one after another, the matrix cores
 // were busy 25% and the VALU 46%, at 2.7 TB/s.
 //

@@ -38,9 +38,9 @@
 // Steps past a wave's range load through a resource of zero records (zeros, no traffic) and
 // their scales are masked to zero, so any K that is a multiple of 64 runs.
 //
-// Measured (us a launch, distinct weights, before -> after): [14336,4096] 4-bit 32 rows
-// 19.5 -> 15.5, 64 rows 37 -> 20.5, 77 rows 54 -> 23, 128 rows 54 -> 27.5; 8-bit 64 rows
-// 45 -> 27, 128 rows 57 -> 31.5.
+// Measured (us a call, distinct weights, before -> after): [14336,4096] 4-bit 32 rows
+// 19.5 -> 15.5, 64 rows 37 -> 20.5, 77 rows 54 -> 23, 128 rows 42.3 -> 26.7; 8-bit 64 rows
+// 45 -> 27, 128 rows 42.9 -> 30.1. At 77 rows the matrix cores are busy 16% and the VALU 17%.
 #pragma once
 #include "mi_common.h"
 #include "qmv_common.h"

@@ -17,8 +17,8 @@
 // 16x16x32 sustains 1.96 PF and 32x32x16 1.70 PF (registers only, all CUs; 2.4 and 2.3 PF on
 // zeros), so the smaller shape is taken; with the accumulators in plain VGPRs, since in AGPRs
 // the compiler copied them around these MFMAs (4 moves each). 8192 rows 4-bit, 32x32x16 ->
-// 16x16x32: [14336,4096] 889 -> 805 us, [4096,14336] 822 -> 759 (matrix cores busy 60% / 63% at
-// 1.91 GHz, before 59% / 64% at 1.74).
+// 16x16x32: [14336,4096] 889 -> 805 us, [4096,14336] 822 -> 759 (matrix cores busy 59% / 62% of the
+// cycles, before 59% / 64% at a lower clock).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>

@@ -175,8 +175,9 @@ __global__ void __launch_bounds__(256) dequant4_bf16_kernel(u32x4_t* __restrict_
 // its group is p >> gshift (gs / 8 packs). What bounds it is HBM: [14336,4096] 6-bit 44 MB
 // in and 117 MB out; with the GEMM behind it 256 rows fell from 146 to 83 us (fp modes 141-158
 // to 78-84) against a thread a pack or word with byte loads and 2-byte stores.
-// Scale bytes whose products the conversions do not give exactly (e8m0 below 8 or 255, zero
-// e4m3) take the element decoders, as every call with fp32 output or a global scale does.
+// The element decoders, as every call with fp32 output or a global scale, serve e8m0 255 (infinity:
+// NaN from the conversions), e8m0 below 8 (results outside bf16's normal range, where the
+// conversions proved exact too) and zero e4m3 scales (the sign of zero).
 template <int FMT, bool OPWISE>
 __global__ void __launch_bounds__(256) dequant_packs_kernel(u32x4_t* __restrict__ out,
                                                            const uint32_t* __restrict__ w,
